@@ -8,11 +8,12 @@
 // output columns of one row per accumulator quad, which the epilogue stores
 // as one 8-byte write after bias, GELU and residual.
 //
-// Two kernels: gemm_dma_kernel (256 x 256 tiles, 8 waves, global->LDS
-// streaming; the last K step masked when K is not a multiple of 64) for every
-// GEMM of the block and the rollout, plain or with a fused epilogue, and
-// gemm_bias_act_kernel (128 x 128 tiles, register-staged loads) for row
-// strides too long for the former's 32-bit lane offsets.
+// Three kernels: gemm_dma_kernel (256 x 256 tiles, 8 waves, global->LDS
+// streaming; the last K step masked when K is not a multiple of 64) wherever
+// its tiles fill the chip, gemm_tile_kernel (128 x 128 or 64 x 64 tiles,
+// several workgroups per CU) where they do not, and gemm_bias_act_kernel
+// (128 x 128 tiles, register-staged loads) for row strides too long for the
+// former's 32-bit lane offsets.
 #include "gemm.h"
 
 namespace strata {
@@ -731,6 +732,217 @@ __global__ __launch_bounds__(512, 1) void gemm_dma_kernel(GemmParams p) {
   gemm_dma_body<256, 256, 2, 4, 64, 2, ACT, RES, SAVE, KTAIL>(p);
 }
 
+// ---------------------------------------------------------------------------
+// Smaller tiles, for products whose 256 x 256 tiles leave CUs idle.
+// One BM x BN tile per workgroup of WGM x WGN waves; the stages of BK = 64
+// columns stream through an NST-slot LDS ring, NST - 1 stages ahead of the
+// MFMAs (a counted vmcnt wait leaves the younger stages' copies in flight).
+// Bound by the copies: a tile of half the edge moves twice the bytes per MFMA,
+// so these lose to the 256 x 256 kernel wherever that one fills the chip.
+// The MFMA, the K order and the bias as the first C operand are those of
+// gemm_dma_body, so the two agree bit for bit and the choice of a tile (which
+// depends on M) never shows in a result.  Activation, residual mode and the
+// ragged last stage are uniform run-time branches: one instance per tile.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int WGM, int WGN, int NST>
+__global__ __launch_bounds__(64 * WGM * WGN) void gemm_tile_kernel(GemmParams p) {
+  constexpr int BK = 64, NW = WGM * WGN;
+  constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 32, FN = WTN / 32;
+  constexpr int ROWB = BK * 2, CH = ROWB / 16, RPC = 1024 / ROWB;
+  constexpr int XB = BM * ROWB, XCH = XB / 1024, STAGE = XB + BN * ROWB;
+  constexpr int LPW = STAGE / 1024 / NW;
+  constexpr int SLAB = WTM * WTN * 2;  // one wave's epilogue slab: its whole tile in bf16
+  static_assert(WTM % 32 == 0 && WTN % 32 == 0 && XCH % NW == 0 && (STAGE / 1024) % NW == 0, "wave tile / stage layout");
+  static_assert(NW * SLAB <= NST * STAGE, "the epilogue slabs fit the ring");
+  __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE];
+
+  const int tid = (int)__builtin_amdgcn_workitem_id_x();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave / WGN, wn = wave % WGN, l32 = lane & 31, hi = lane >> 5;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+
+  // Tiles in groups of 8 row panels x every column panel, row panel fastest, an
+  // XCD-contiguous run of them per XCD (its L2 holds the run's panels).
+  int64_t m0, n0;
+  {
+    const int wg = xcd_tile_order(p.mt * p.nt, (int)__builtin_amdgcn_workgroup_id_x());
+    constexpr int GRP = 8;
+    const int gi = wg / (GRP * p.nt), li = wg % (GRP * p.nt), gmn = min(GRP, p.mt - gi * GRP);
+    m0 = (int64_t)(gi * GRP + li % gmn) * BM;
+    n0 = (int64_t)(li / gmn) * BN;
+  }
+
+  // Copy j of a stage fills rows RPC * c .. of the x tile (c = j * NW + wave < XCH)
+  // or of the w tile; rows past M (N) read as zero.
+  uint32_t voff[LPW];
+#pragma unroll
+  for (int j = 0; j < LPW; ++j) {
+    const bool isw = j * NW >= XCH;
+    const int c = j * NW + wave - (isw ? XCH : 0), row = RPC * c + lane / CH;
+    const bool ok = (isw ? n0 : m0) + row < (isw ? p.N : p.M);
+    voff[j] = ok ? (uint32_t)(row * (isw ? p.ldw : p.ldx) * 2 + gswz<CH>(lane % CH, row) * 16) : OOB;
+  }
+  const int nk = (int)((p.K + BK - 1) / BK), ktail = (int)(p.K % BK);
+  const char* xk = (const char*)(p.x + m0 * p.ldx);
+  const char* wk = (const char*)(p.w + n0 * p.ldw);
+  auto issue = [&](int kt, int slot) {
+    const u32x4 rx = make_rsrc(xk + (int64_t)kt * BK * 2, OOB), rw = make_rsrc(wk + (int64_t)kt * BK * 2, OOB);
+    const uint32_t dst = lds_base + slot * STAGE + wave * 1024;
+    const bool last = ktail && kt == nk - 1;  // uniform: chunks at or past K read as zero
+#pragma unroll
+    for (int j = 0; j < LPW; ++j) {
+      const bool isw = j * NW >= XCH;
+      uint32_t vo = voff[j];
+      if (last) {
+        const int row = RPC * (j * NW + wave - (isw ? XCH : 0)) + lane / CH;
+        if (gswz<CH>(lane % CH, row) * 8 >= ktail) vo = OOB;
+      }
+      dma_row16(isw ? rw : rx, dst + j * NW * 1024, vo);
+    }
+  };
+
+  // The bias as the accumulators' first C operand (columns 8q + 4hi + e of each 32).
+  const int64_t gn0 = n0 + wn * WTN, gm0 = m0 + wm * WTM;
+  f32x16 acc[FN][FM];
+  {
+    u32x2 bb[FN][4];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        // N is a multiple of 8: a quad lies inside the matrix or outside it
+        const int64_t gn = min(gn0 + 32 * i + 8 * q + 4 * hi, p.N - 4);
+        bb[i][q] = p.bias ? *(const u32x2*)(p.bias + gn) : (u32x2){0u, 0u};
+      }
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) {
+          acc[i][j][4 * q + 0] = bf16_lo(bb[i][q][0]);
+          acc[i][j][4 * q + 1] = bf16_hi(bb[i][q][0]);
+          acc[i][j][4 * q + 2] = bf16_lo(bb[i][q][1]);
+          acc[i][j][4 * q + 3] = bf16_hi(bb[i][q][1]);
+        }
+  }
+
+  uint32_t aoff[FN][2], boff[FM][2];  // sub-steps 2, 3 flip bit 2 of the chunk: offset ^ 64
+#pragma unroll
+  for (int i = 0; i < FN; ++i) {
+    const int row = wn * WTN + 32 * i + l32;
+    for (int kk = 0; kk < 2; ++kk) aoff[i][kk] = XB + row * ROWB + gswz<CH>(2 * kk + hi, row) * 16;
+  }
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int row = wm * WTM + 32 * j + l32;
+    for (int kk = 0; kk < 2; ++kk) boff[j][kk] = row * ROWB + gswz<CH>(2 * kk + hi, row) * 16;
+  }
+
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nk) issue(s, s);
+  int rd = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // stage kt has landed once at most the NST - 2 younger stages are in flight
+    // (near the end there are fewer: wait for all)
+    if (NST > 2 && kt + NST - 2 < nk) wait_vmcnt((NST - 2) * LPW);
+    else wait_vmcnt(0);
+    lds_barrier();  // landed for every wave, and the slot read last step is free
+    const int wr = rd == 0 ? NST - 1 : rd - 1;
+    if (kt + NST - 1 < nk) issue(kt + NST - 1, wr);
+    const char* st = lds + rd * STAGE;
+    rd = rd + 1 == NST ? 0 : rd + 1;
+    bf16x8 af[2][FN], bfr[2][FM];
+    auto load_frags = [&](int kk, int buf) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i) af[buf][i] = *(const bf16x8*)(st + (aoff[i][kk & 1] ^ ((kk >> 1) * 64)));
+#pragma unroll
+      for (int j = 0; j < FM; ++j) bfr[buf][j] = *(const bf16x8*)(st + (boff[j][kk & 1] ^ ((kk >> 1) * 64)));
+    };
+    load_frags(0, 0);
+#pragma unroll
+    for (int kk = 0; kk < BK / 16; ++kk) {
+      const int cb = kk & 1;
+      if (kk + 1 < BK / 16) load_frags(kk + 1, cb ^ 1);
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cb][i], bfr[cb][j], acc[i][j], 0, 0, 0);
+    }
+  }
+
+  // ---- epilogue: bf16 through this wave's LDS slab, 16-byte rows out ----
+  lds_barrier();  // every wave is done reading the ring
+  constexpr int SRB = WTN * 2, CPR = WTN / 8, RPI = 64 / CPR, NIT = WTM / RPI;
+  char* slab = lds + wave * SLAB;
+  const int c = lane % CPR;
+  const int64_t gn = gn0 + 8 * c;
+  const bool col = gn < p.N;  // N is a multiple of 8: the whole 16-byte run
+  auto to_slab = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int nl = 32 * i + 8 * q + 4 * hi;
+#pragma unroll
+        for (int j = 0; j < FM; ++j) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = f(acc[i][j][4 * q + e]);
+          const int ml = 32 * j + l32;
+          const u32x2 w2 = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          *(u32x2*)(slab + ml * SRB + (((nl >> 3) ^ (ml & (CPR - 1))) << 4) + 8 * hi) = w2;
+        }
+      }
+  };
+  auto from_slab = [&](bf16* dst, auto res) {
+    constexpr int RES = decltype(res)::value;
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      const int sl = RPI * it + lane / CPR;
+      const int64_t gm = gm0 + sl;
+      if (col && gm < p.M) {
+        u32x4 o = *(const u32x4*)(slab + sl * SRB + ((c ^ (sl & (CPR - 1))) << 4));
+        if constexpr (RES != RES_NONE_T) {
+          const u32x4 r = *(const u32x4*)(p.res + gm * p.ldr + gn);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            o[e] = pack_bf16x2(combine_t<RES>(bf16_lo(o[e]), bf16_lo(r[e])),
+                               combine_t<RES>(bf16_hi(o[e]), bf16_hi(r[e])));
+        }
+        *(u32x4*)(dst + gm * p.ldo + gn) = o;
+      }
+    }
+  };
+  switch (p.act) {
+    case STRATA_HIP_ACT_GELU_TANH: to_slab([](float x) { return gelu_tanh(x); }); break;
+    case STRATA_HIP_ACT_GELU_ERF: to_slab([](float x) { return gelu_erf(x); }); break;
+    case STRATA_HIP_ACT_SIGMOID: to_slab([](float x) { return sigmoid_fast(x); }); break;
+    case STRATA_HIP_ACT_GELU_TANH_GRAD: to_slab([](float x) { return gelu_tanh_grad(x); }); break;
+    case STRATA_HIP_ACT_SIGMOID_GRAD: to_slab([](float x) { return sigmoid_grad(x); }); break;
+    default: to_slab([](float x) { return x; }); break;
+  }
+  if (!p.res) from_slab(p.out, std::integral_constant<int, RES_NONE_T>{});
+  else if (p.res_op == STRATA_HIP_RES_MUL) from_slab(p.out, std::integral_constant<int, RES_MUL_T>{});
+  else from_slab(p.out, std::integral_constant<int, RES_ADD_T>{});
+  if (p.out2) {  // the saved derivative (GELU(tanh), no residual)
+    to_slab([](float x) { return gelu_tanh_grad(x); });
+    from_slab(p.out2, std::integral_constant<int, RES_NONE_T>{});
+  }
+}
+
+template <int BM, int BN, int WGM, int WGN, int NST>
+static int launch_tile(GemmParams p, hipStream_t st) {
+  p.mt = (int)((p.M + BM - 1) / BM);
+  p.nt = (int)((p.N + BN - 1) / BN);
+  const int64_t total = (int64_t)p.mt * p.nt;
+  if (total > 0x7fffffff) return fail(STRATA_HIP_EUNSUPPORTED, "gemm: problem too large for one launch");
+  hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NST>), dim3((unsigned)total), dim3(64 * WGM * WGN), 0, st, p);
+  return check_launch("gemm_tile_kernel");
+}
+
 template <int ACT>
 static void launch_dma_act(const GemmParams& p, dim3 grid, hipStream_t st) {
   auto go = [&](auto ktail) {
@@ -811,19 +1023,66 @@ static int gemm_params(const strata_hip_gemm_args* a, GemmParams& p) {
   return STRATA_HIP_OK;
 }
 
-// The large-tile kernel streams 64-wide K steps (the last one masked when K
-// is not a multiple of 64) with 32-bit lane offsets inside a 256-row block:
-// row strides small enough.
-// Sets the tile counts; the persistent grid is one workgroup per CU (the
-// 128 KiB ring admits one).
-static bool gemm_big(GemmParams& p, dim3& grid) {
-  if (!(256 * p.ldx * 2 + 4096 < (int64_t)OOB && 256 * p.ldw * 2 + 4096 < (int64_t)OOB)) return false;
+// The DMA kernels stream 64-wide K steps (the last one masked when K is not a
+// multiple of 64) with 32-bit lane offsets inside a 256-row block: row strides
+// small enough.
+static bool gemm_dma_ok(const GemmParams& p) {
+  return 256 * p.ldx * 2 + 4096 < (int64_t)OOB && 256 * p.ldw * 2 + 4096 < (int64_t)OOB &&
+         ((p.M + 255) / 256) * ((p.N + 255) / 256) <= 0x7fffffff;
+}
+
+// Sets the 256 x 256 kernel's tile counts; its persistent grid is one workgroup
+// per CU (the 128 KiB ring admits one).
+static dim3 gemm_big(GemmParams& p) {
   p.mt = (int)((p.M + 255) / 256);
   p.nt = (int)((p.N + 255) / 256);
   const int64_t total = (int64_t)p.mt * p.nt;
   const int cus = device_cus();
-  grid = dim3((unsigned)(total < cus ? total : cus));
-  return total <= 0x7fffffff;
+  return dim3((unsigned)(total < cus ? total : cus));
+}
+
+// Which tile a product takes: the least estimated time.  A round is one tile in
+// every slot (CUs x workgroups per CU); per K it takes t0 ns nearly alone and t1
+// ns with the chip full (the copies then compete for L2), plus the epilogue:
+//   256 x 256           1 per CU   16.5 .. 26 ns    5.0 us   (whole rounds: persistent)
+//   128 x 128           2 per CU    8.3 .. 17.9     3.7
+//   128 x 128, 3 slots  1 per CU    7   .. 9.6      3        (for one round: a deeper ring)
+//   64 x 64             2 per CU    5   .. 7        1.6
+// fitted on 40 shapes; the estimate picks the fastest of the four or one within
+// ~10% of it.  Measured, us, 256 x 256 only -> the choice: M x N x K =
+// 1024 x 256 x 1024 24.0 -> 7.6 (64 x 64), 2000 x 1024 x 4096 76 -> 28 (64 x 64),
+// 3040 x 888 x 3552 75 -> 34 (3 slots), 10125 x 768 x 3072 61 -> 52 (128 x 128),
+// 65536 x 128 x 128 15.9 -> 11.2 (128 x 128); at 49152 x 1024 x 4096 the 256 x 256
+// kernel's 326 stand against 440 and 695.
+enum GemmTile { TILE_256, TILE_128, TILE_128_DEEP, TILE_64 };
+static GemmTile gemm_choose(const GemmParams& p) {
+  if (p.N % 8) return TILE_256;  // the smaller tiles store whole 16-byte runs
+  const double K = (double)p.K, cus = device_cus();
+  auto tiles = [&](int64_t b) { return (double)(((p.M + b - 1) / b) * ((p.N + b - 1) / b)); };
+  const double r256 = tiles(256) / cus, whole = (double)(int64_t)r256, part = r256 - whole;
+  double best = 3000. + whole * (26. * K + 5000.) + (part > 0. ? (16.5 + 9.5 * part) * K + 5000. : 0.);
+  GemmTile pick = TILE_256;
+  auto offer = [&](GemmTile t, double ns) {
+    if (ns < best) {
+      best = ns;
+      pick = t;
+    }
+  };
+  const double r128 = tiles(128) / (2. * cus), r64 = tiles(64) / (2. * cus);
+  offer(TILE_128, r128 > 1. ? 3000. + r128 * (17.9 * K + 3700.) : 4000. + (8.3 + 9.6 * r128) * K);
+  if (r128 <= .5) offer(TILE_128_DEEP, 3000. + (7. + 5.2 * r128) * K);
+  offer(TILE_64, r64 > 1. ? 2000. + r64 * (7.05 * K + 1600.) : 2000. + (5. + 2. * r64) * K);
+  return pick;
+}
+
+// The smaller tiles, where one of them is chosen; 1: the 256 x 256 kernel.
+static int gemm_small(const GemmParams& p, hipStream_t st) {
+  switch (gemm_choose(p)) {
+    case TILE_128: return launch_tile<128, 128, 4, 2, 2>(p, st);
+    case TILE_128_DEEP: return launch_tile<128, 128, 4, 2, 3>(p, st);
+    case TILE_64: return launch_tile<64, 64, 2, 2, 4>(p, st);
+    default: return 1;
+  }
 }
 
 }  // namespace strata
@@ -833,8 +1092,9 @@ extern "C" int strata_hip_gemm_bias_act(const strata_hip_gemm_args* a, void* str
   if (const int rc = gemm_params(a, p)) return rc;
   if (a->m == 0 || a->n == 0) return STRATA_HIP_OK;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid;
-  if (gemm_big(p, grid)) {
+  if (gemm_dma_ok(p)) {
+    if (const int rc = gemm_small(p, st); rc <= 0) return rc;
+    const dim3 grid = gemm_big(p);
     switch (p.act) {
       case STRATA_HIP_ACT_GELU_TANH: launch_dma_act<STRATA_HIP_ACT_GELU_TANH>(p, grid, st); break;
       case STRATA_HIP_ACT_GELU_ERF: launch_dma_act<STRATA_HIP_ACT_GELU_ERF>(p, grid, st); break;
@@ -856,9 +1116,10 @@ extern "C" int strata_hip_gemm_gelu_save(const strata_hip_gemm_args* a, void* da
   if (a->m == 0 || a->n == 0) return STRATA_HIP_OK;
   if (!dact || ((uintptr_t)dact & 7)) return fail(STRATA_HIP_EINVAL, "gemm_gelu_save: dact must be 8-byte aligned");
   p.out2 = (bf16*)dact;
-  dim3 grid;
-  if (!gemm_big(p, grid))
+  if (!gemm_dma_ok(p))
     return fail(STRATA_HIP_EUNSUPPORTED, "gemm_gelu_save: row strides too long for the large-tile kernel");
+  if (const int rc = gemm_small(p, (hipStream_t)stream); rc <= 0) return rc;
+  const dim3 grid = gemm_big(p);
   if (p.K % 64)
     hipLaunchKernelGGL((gemm_dma_kernel<STRATA_HIP_ACT_GELU_TANH, RES_NONE_T, true, true>), grid, dim3(512), 0,
                        (hipStream_t)stream, p);

@@ -396,3 +396,47 @@ def test_ops_reject_cpu_tensors(gpu):
     x = torch.zeros(4, 64, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="GPU"):
         torch.ops.strata_hip.layer_norm(x, 1e-6)
+
+
+# (M, N, K): the smaller tiles' edges (one token, 64 and 128 and their neighbours), ragged
+# last columns and K stages, and each of the four tiles by the sizes that choose it
+TILE_SHAPES = [(1, 8, 8), (63, 64, 64), (65, 72, 72), (128, 256, 256), (129, 136, 520), (1350, 104, 208),
+               (1024, 256, 1024), (2000, 1024, 4096), (3040, 888, 3552), (10125, 768, 768)]
+
+
+@pytest.mark.parametrize("shape", TILE_SHAPES, ids=str)
+@pytest.mark.parametrize("act,res_op", [(_lib.ACT_NONE, None), (_lib.ACT_NONE, _lib.RES_ADD), (_lib.ACT_GELU_TANH, None),
+                                        (_lib.ACT_SIGMOID, _lib.RES_MUL), (_lib.ACT_GELU_TANH_GRAD, _lib.RES_MUL),
+                                        (_lib.ACT_GELU_ERF, None)])
+def test_gemm_smaller_tiles(gpu, shape, act, res_op):
+    """Products whose 256 x 256 tiles would leave CUs idle, against float64 (bf16 rounding of
+    the activation and of the sum: 2^-8 each, so 1e-2), and bit for bit against the same rows
+    inside a product large enough for the 256 x 256 tiles: the tile never shows in a result."""
+    M, N, K = shape
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w, b, r = (torch.randn(s, generator=g).bfloat16() for s in ((M, K), (N, K), (N,), (M, N)))
+    w = (w.float() * K**-0.5).bfloat16()
+    res = r if res_op is not None else None
+    on = lambda t: t.to(gpu) if t is not None else None  # noqa: E731
+    got = ops.gemm_bias_act(on(x), on(w), on(b), on(res), act, res_op or 0)
+    z = x.double() @ w.double().T + b.double()
+    ref = {_lib.ACT_NONE: lambda t: t, _lib.ACT_SIGMOID: torch.sigmoid,
+           _lib.ACT_GELU_TANH: lambda t: F.gelu(t, approximate="tanh"), _lib.ACT_GELU_ERF: F.gelu,
+           _lib.ACT_GELU_TANH_GRAD: lambda t: _gelu_tanh_grad(t)}[act](z)
+    if res_op is not None:
+        ref = ref + r.double() if res_op == _lib.RES_ADD else ref * r.double()
+    assert rel_l2(got.float().cpu(), ref.float()) <= 1e-2
+    big = 70000  # rows: 256 x 256 tiles fill the chip at every N and K above
+    if act == _lib.ACT_NONE:
+        xb = torch.cat([on(x), torch.zeros(big - M, K, dtype=torch.bfloat16, device=gpu)])
+        rb = torch.cat([on(res), torch.zeros(big - M, N, dtype=torch.bfloat16, device=gpu)]) if res is not None else None
+        n = -(-N // 1024) * 1024  # and columns
+        wb = torch.cat([on(w), torch.zeros(n - N, K, dtype=torch.bfloat16, device=gpu)])
+        bb = torch.cat([on(b), torch.zeros(n - N, dtype=torch.bfloat16, device=gpu)])
+        rb = F.pad(rb, (0, n - N)) if rb is not None else None
+        assert torch.equal(ops.gemm_bias_act(xb, wb, bb, rb, act, res_op or 0)[:M, :N], got)
+
+
+def _gelu_tanh_grad(t):
+    t = t.clone().requires_grad_(True)
+    return torch.autograd.grad(F.gelu(t, approximate="tanh").sum(), t)[0]
