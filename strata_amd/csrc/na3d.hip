@@ -3,8 +3,8 @@
 // Semantics follow NATTEN's na3d (0.21.5): clamped windows, optional dilation,
 // non-causal, softmax over kz*ky*kx keys scaled by `scale`.  Three kernels:
 //
-//  * na3d_scalar_kernel: one thread per (batch, query, head), fp32 math, used
-//    for fp32 inputs and for shapes the MFMA kernel does not cover.
+//  * na3d_scalar_kernel: one thread per (batch, query, head), fp32 math, for
+//    shapes neither the MFMA kernels nor (fp32 inputs) na3d_gather.hip cover.
 //  * na3d_mfma_kernel:   bf16 inputs, fp32 accumulation.  A workgroup owns a
 //    (1, NTY*TY, 4*TX) box of queries of one (batch, head, dilation residue);
 //    each of its 4 waves owns NTY tiles of (TY, TX) = 16 queries stacked in y.
@@ -24,6 +24,7 @@
 #include <utility>
 
 #include "common.h"
+#include "na3d_gather.h"
 
 namespace strata {
 
@@ -2304,6 +2305,35 @@ static int launch_scalar(const Na3dParams& p, hipStream_t st) {
   return check_launch("na3d_scalar_kernel");
 }
 
+// fp32 tensors: the gather kernel on the matrix cores, else one thread per query.
+static int launch_f32(const Na3dParams& p, hipStream_t st) {
+  GatherParams g = {};
+  g.c0 = p.q;
+  g.s0 = p.k;
+  g.s1 = p.v;
+  g.o0 = p.o;
+  g.B = p.B;
+  g.H = p.H;
+  g.D = p.D;
+  for (int a = 0; a < 3; ++a) {
+    g.L[a] = p.L[a];
+    g.org[a] = p.org[a];
+    g.ext[a] = p.ext[a];
+    g.ker[a] = p.ker[a];
+    g.dil[a] = p.dil[a];
+  }
+  for (int i = 0; i < 5; ++i) {
+    g.cs[i] = p.qs[i];
+    g.ss0[i] = p.ks[i];
+    g.ss1[i] = p.vs[i];
+    g.os[i] = p.os[i];
+  }
+  g.scale = p.scale;
+  g.lse = p.lse;
+  g.lse_ext1 = p.lse_ext1;
+  return gather_fits(g, GATHER_FWD, 4) ? launch_gather(g, GATHER_FWD, false, st) : launch_scalar<float>(p, st);
+}
+
 // Query counts per axis of the box (largest over the dilation residue classes).
 static void box_queries(const Na3dParams& p, int (&nq)[3]) {
   for (int a = 0; a < 3; ++a) {
@@ -2737,7 +2767,7 @@ extern "C" int strata_hip_na3d_fwd(const strata_hip_na3d_args* a, void* stream) 
   if (const int rc = na3d_prepare(a, p)) return rc;
   if ((int64_t)p.B * p.ext[0] * p.ext[1] * p.ext[2] == 0) return STRATA_HIP_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (a->dtype == STRATA_HIP_F32) return launch_scalar<float>(p, st);
+  if (a->dtype == STRATA_HIP_F32) return launch_f32(p, st);
   const bool mfma_ok = na3d_mfma_ok(p);
   if (!mfma_ok) return launch_scalar<bf16>(p, st);
   if (column_fits(p)) return launch_column(p, st);

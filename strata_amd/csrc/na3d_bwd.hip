@@ -13,9 +13,11 @@
 // workgroup's shared K/V or Q/dO rows in LDS; for ky in {5, 7}, kx <= 9,
 // kz >= 3 (the block's windows) dq, dV and dK walk strips like the forward
 // (the rows whose windows are not clamped) and the clamped edge rows walk
-// tiles, all in one launch (na3d_bwd_small_fused_kernel).  The general VALU
-// versions (4 lanes per token, D/4 head dims per lane, dot products closed by
-// two xor shuffles) take everything else:
+// tiles, all in one launch (na3d_bwd_small_fused_kernel).  fp32, other head
+// dims, dilation and wider windows run na3d_gather.hip's fp32-arithmetic MFMA
+// kernels; the general VALU versions (4 lanes per token, D/4 head dims per lane,
+// dot products closed by two xor shuffles) take what those refuse and the prep
+// without a forward lse:
 //   prep: per query, log2-sum-exp of its scores (recomputed, unless the caller
 //         passes the forward's, strata_hip_na3d_fwd's lse output: then only
 //         D_i) and D_i, into a caller-provided fp32 workspace;
@@ -31,6 +33,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "na3d_gather.h"
 
 namespace strata {
 
@@ -1601,6 +1604,34 @@ static void launch_dq_strips(const Na3dBwdParams& p, const BwdStrips& sg, hipStr
   }
 }
 
+// The fp32-arithmetic MFMA kernels over the whole grid (contiguous tensors).
+static GatherParams bwd_gather(const Na3dBwdParams& p, int D, int mode) {
+  GatherParams g = {};
+  const bool dkv = mode == GATHER_DKV;
+  g.c0 = dkv ? p.k : p.q;
+  g.c1 = dkv ? p.v : p.dout;
+  g.s0 = dkv ? p.q : p.k;
+  g.s1 = dkv ? p.dout : p.v;
+  g.o0 = dkv ? p.dk : p.dq;
+  g.o1 = dkv ? p.dv : nullptr;
+  g.B = p.B;
+  g.H = p.H;
+  g.D = D;
+  const int L[3] = {p.Z, p.Y, p.X};
+  for (int a = 0; a < 3; ++a) {
+    g.L[a] = g.ext[a] = L[a];
+    g.ker[a] = p.ker[a];
+    g.dil[a] = p.dil[a];
+  }
+  const int64_t hd = (int64_t)p.H * D;
+  const int64_t s[5] = {hd * p.X * p.Y * p.Z, hd * p.X * p.Y, hd * p.X, hd, D};
+  for (int i = 0; i < 5; ++i) g.cs[i] = g.ss0[i] = g.ss1[i] = g.os[i] = s[i];
+  g.scale = p.scale;
+  g.lse = p.lse;
+  g.dsum = p.dsum;
+  return g;
+}
+
 template <typename T, int D>
 static int launch_bwd(const Na3dBwdParams& p, hipStream_t st) {
   const int64_t blocks = (int64_t)p.B * p.H * p.Z * p.nyt * p.nxt;
@@ -1616,6 +1647,13 @@ static int launch_bwd(const Na3dBwdParams& p, hipStream_t st) {
     hipLaunchKernelGGL(na3d_bwd_prep_mfma_kernel, grid, block, 0, st, p);
   } else {
     hipLaunchKernelGGL((na3d_bwd_prep_kernel<T, D>), grid, block, 0, st, p);
+  }
+  if (!(sizeof(T) == 2 && D == 64 && mfma_ok(p)) && !std::getenv("STRATA_HIP_NA3D_BWD_VALU")) {
+    const GatherParams gq = bwd_gather(p, D, GATHER_DQ), gkv = bwd_gather(p, D, GATHER_DKV);
+    if (gather_fits(gq, GATHER_DQ, sizeof(T)) && gather_fits(gkv, GATHER_DKV, sizeof(T))) {
+      if (const int rc = launch_gather(gq, GATHER_DQ, sizeof(T) == 2, st)) return rc;
+      return launch_gather(gkv, GATHER_DKV, sizeof(T) == 2, st);
+    }
   }
   // LDS kernels: workgroups of 4 * NT rows
   constexpr int NT = NA3D_BWD_NT;

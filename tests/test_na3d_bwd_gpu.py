@@ -211,3 +211,44 @@ def test_bwd_with_forward_lse_matches_recompute(gpu, case):
         assert rel_l2(a.float().cpu(), r) <= 1e-2, name
         assert rel_l2(b.float().cpu(), r) <= 1e-2, name
         assert rel_l2(a.float(), b.float()) <= 4e-3, name
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 1e-2)], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("grid,H,D,kernel,dil", [
+    ((1, 3, 3), 1, 32, (1, 3, 3), (1, 1, 1)),
+    ((4, 9, 10), 2, 128, (3, 5, 5), (1, 1, 1)),   # every axis clamped
+    ((5, 13, 15), 2, 32, (3, 5, 3), (1, 2, 3)),   # unequal residue classes
+    ((6, 11, 17), 2, 64, (3, 3, 15), (1, 1, 1)),  # wider than the LDS kernels take
+    ((4, 30, 33), 4, 128, (3, 7, 7), (1, 1, 1)),
+    ((8, 18, 18), 1, 32, (7, 9, 9), (1, 1, 1)),   # more rows than one table holds
+], ids=str)
+def test_bwd_gather_kernels(gpu, grid, H, D, kernel, dil, dtype, tol):
+    """The fp32-arithmetic MFMA backward (fp32; bf16 with other head dims, dilation or wide
+    windows) against the float64 oracle's gradients, tolerances as the tests above."""
+    g = torch.Generator().manual_seed(9)
+    q, k, v, do = (torch.randn((2, *grid, H, D), generator=g).to(dtype) for _ in range(4))
+    ref = O.na3d_backward(q, k, v, do, kernel, dil, compute_dtype=torch.float64)
+    out, lse = ops.na3d_fwd_lse(q.to(gpu), k.to(gpu), v.to(gpu), list(kernel), list(dil), None)
+    got = ops.na3d_bwd(q.to(gpu), k.to(gpu), v.to(gpu), out, do.to(gpu), list(kernel), list(dil), None, lse)
+    for name, a, b in zip(("dq", "dk", "dv"), got, ref):
+        assert rel_l2(a.float().cpu(), b) <= tol, name
+
+
+def test_bwd_gather_kernels_keep_non_finite_values_inside_their_windows(gpu):
+    """A NaN output gradient at one query reaches dk and dv of exactly its window's keys."""
+    g = torch.Generator().manual_seed(10)
+    q, k, v, do = (torch.randn((1, 3, 10, 11, 2, 32), generator=g).to(gpu) for _ in range(4))
+    kernel, at = [3, 5, 5], (0, 1, 4, 2, 0)
+    out, lse = ops.na3d_fwd_lse(q, k, v, kernel, [1, 1, 1], None)
+    clean = ops.na3d_bwd(q, k, v, out, do, kernel, [1, 1, 1], None, lse)
+    bad = do.clone()
+    bad[at] = float("nan")
+    got = ops.na3d_bwd(q, k, v, out, bad, kernel, [1, 1, 1], None, lse)
+    held = torch.zeros(1, 3, 10, 11, 2, dtype=torch.bool, device=gpu)
+    held[0, :, 2:7, 0:5, 0] = True  # the window of (1, 4, 2)
+    for a, c in zip(got[1:], clean[1:]):
+        # the affected blocks sum in another order: fp32 rounding apart
+        assert torch.isnan(a[held]).all() and (a[~held] - c[~held]).abs().max().item() <= 1e-5
+    one = torch.zeros_like(held)
+    one[at] = True
+    assert torch.isnan(got[0][one]).all() and (got[0][~one] - clean[0][~one]).abs().max().item() <= 1e-5

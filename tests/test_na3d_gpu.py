@@ -406,3 +406,64 @@ def test_depthwise_lse_and_strided_views(gpu):
     ref, ref_lse = O.na3d(q, k, v, (Z, 1, 1), compute_dtype=torch.float64, return_lse=True)
     assert rel_l2(out.float(), ref) <= BF16_TOL
     assert (lse.double().cpu() - ref_lse).abs().max().item() <= 2e-2
+
+
+# grid, heads, head_dim, kernel, dilation, query box: tile remainders on every axis, each split
+# of a tile over waves (few tiles), a window as long as its axis, dilated residue classes with
+# unequal counts, a column window, and more rows than one table holds (8 x 14 x 14 > 512)
+GATHER_CASES = [
+    ((1, 3, 3), 1, 32, (1, 3, 3), (1, 1, 1), None),
+    ((4, 17, 19), 3, 64, (3, 5, 7), (1, 1, 1), None),
+    ((5, 11, 13), 2, 128, (3, 3, 3), (1, 2, 3), None),
+    ((9, 16, 21), 2, 32, (7, 11, 11), (1, 1, 1), None),
+    ((6, 14, 15), 2, 64, (6, 1, 1), (1, 1, 1), None),
+    ((3, 24, 30), 2, 64, (3, 9, 5), (1, 1, 2), ((0, 3, 5), (3, 17, 19))),
+    ((4, 40, 44), 8, 32, (3, 7, 7), (1, 1, 1), None),
+]
+
+
+@pytest.mark.parametrize("strided", [False, True], ids=["contiguous", "packed"])
+@pytest.mark.parametrize("case", GATHER_CASES, ids=str)
+def test_fp32_gather_kernel(gpu, case, strided):
+    """fp32 NA3D on the matrix cores against the float64 oracle (<= 1e-5, as every fp32 case),
+    its log2-sum-exp, and q, k, v as views of one packed qkv buffer."""
+    grid, H, D, kernel, dil, box = case
+    q, k, v = _rand((2, *grid, H, D), 5, torch.float32, gpu)
+    if strided:
+        q, k, v = torch.stack([q, k, v], dim=4).unbind(4)
+    origin, extent = box or ((0, 0, 0), grid)
+    got = _run(q, k, v, kernel, dil, origin, extent)
+    ref, lse = O.na3d(q.cpu(), k.cpu(), v.cpu(), kernel, dil, q_origin=origin, q_extent=extent,
+                      compute_dtype=torch.float64, return_lse=True)
+    assert (got.cpu().double() - ref).abs().max().item() <= F32_TOL
+    if box is None:
+        out, got_lse = torch.ops.strata_hip.na3d_fwd_lse(q, k, v, list(kernel), list(dil), None)
+        assert torch.equal(out, got)
+        assert (got_lse.cpu().double() - lse).abs().max().item() <= 1e-4
+
+
+def test_fp32_gather_kernel_keeps_non_finite_values_inside_their_windows(gpu):
+    """A NaN or infinite value token reaches exactly the queries whose windows hold it; a key of
+    -inf scores carries no weight, and one of +inf or NaN scores makes its queries NaN."""
+    q, k, v = _rand((1, 4, 12, 14, 2, 64), 6, torch.float32, gpu)
+    kernel, at = (3, 5, 5), (0, 1, 6, 3, 1)  # (b, z, y, x, h)
+    clean = _run(q, k, v, kernel)
+    probe = torch.zeros_like(v)
+    probe[at] = 1.0
+    reached = _run(torch.zeros_like(q), k, probe, kernel)[..., 0] > 0  # uniform weights: the windows that hold it
+    for bad in (float("nan"), float("inf"), -float("inf")):
+        vb = v.clone()
+        vb[at] = bad
+        out = _run(q, k, vb, kernel)
+        # the affected blocks sum in another order: fp32 rounding apart
+        assert (out[~reached] - clean[~reached]).abs().max().item() <= F32_TOL
+        assert not torch.isfinite(out[reached]).any()
+    ones = torch.ones_like(q)
+    kb = k.clone()
+    kb[at] = -float("inf")
+    out = _run(ones, kb, v, kernel)
+    ref = _run(ones, torch.where(torch.isfinite(kb), kb, torch.full_like(kb, -1e30)), v, kernel)
+    assert (out - ref).abs().max().item() <= F32_TOL
+    kb[at] = float("nan")
+    out = _run(ones, kb, v, kernel)
+    assert torch.isnan(out[reached]).all() and torch.isfinite(out[~reached]).all()
