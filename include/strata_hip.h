@@ -458,6 +458,15 @@ typedef struct strata_hip_dealias_axis_args {
 
 int strata_hip_dealias_axis(const strata_hip_dealias_axis_args* args, void* stream);
 
+/* strata_hip_dealias_axis along y (when ny > 1) and x (when nx > 1), the input
+ * normalisation in the first of them, and strata_hip_state_patchify of the result,
+ * in one launch and bit for bit as that chain.  taps_y / taps_x: host arrays of ny /
+ * nx taps (1..16; 1: the axis is not filtered).  args as strata_hip_state_patchify;
+ * patch widths (x) 1, 2 and 4, X a multiple of 4 and a 16-byte aligned state, else
+ * STRATA_HIP_EUNSUPPORTED. */
+int strata_hip_dealias_patchify(const strata_hip_state_patchify_args* args, const float* taps_y, int32_t ny,
+                                const float* taps_x, int32_t nx, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Pipeline step, output side: unpatchify of the prediction tokens, the target
  * denormalisation (RunningNorm2d.denormalize, screamcast/normalization.py:102-107)

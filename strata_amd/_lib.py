@@ -335,6 +335,9 @@ EXPORTS = {
     "strata_hip_cube_crop": ([ctypes.POINTER(CubeCropArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_state_patchify": ([ctypes.POINTER(StatePatchifyArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_dealias_axis": ([ctypes.POINTER(DealiasAxisArgs), ctypes.c_void_p], ctypes.c_int),
+    "strata_hip_dealias_patchify": (
+        [ctypes.POINTER(StatePatchifyArgs), ctypes.POINTER(ctypes.c_float), ctypes.c_int32,
+         ctypes.POINTER(ctypes.c_float), ctypes.c_int32, ctypes.c_void_p], ctypes.c_int),
     "strata_hip_state_update": ([ctypes.POINTER(StateUpdateArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_upsample_dw_gelu": ([ctypes.POINTER(UpsampleDwGeluArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_layer_norm_modulate": ([ctypes.POINTER(LayerNormModulateArgs), ctypes.c_void_p], ctypes.c_int),

@@ -35,6 +35,7 @@ __all__ = [
     "cube_crop",
     "state_patchify",
     "dealias_axis",
+    "dealias_patchify",
     "state_update",
     "upsample_dw_gelu",
     "layer_norm_modulate",
@@ -1009,6 +1010,66 @@ def _(state, mean, std, axis, patch, taps):
 
 
 dealias_axis.register_autograd(_no_backward("strata_hip::dealias_axis"))
+
+
+@torch.library.custom_op("strata_hip::dealias_patchify", mutates_args=())
+def dealias_patchify(
+    state: Tensor, mean: Optional[Tensor], std: Optional[Tensor], patch: Sequence[int], taps_y: Sequence[float],
+    taps_x: Sequence[float]
+) -> Tensor:
+    """``state_patchify`` of the state filtered by ``dealias_axis`` along y and x (the input
+    normalisation in the first pass; an axis with one tap is not filtered), bit for bit: one
+    launch for patch widths 1, 2 and 4 and an x extent that is a multiple of 4, else that chain."""
+    name = "dealias_patchify"
+    dev = _require_gpu(name, state)
+    if state.dtype != torch.float32 or state.dim() != 5:
+        raise ValueError(f"{name}: state must be float32 [B, C, Z, Y, X], got {state.dtype} {tuple(state.shape)}")
+    if (mean is None) != (std is None):
+        raise ValueError(f"{name}: give both mean and std, or neither")
+    pz, py, px = _triple("patch", patch)
+    B, C, Z, Y, X = state.shape
+    if min(pz, py, px) <= 0 or Z % pz or Y % py or X % px:
+        raise ValueError(f"{name}: grid {(Z, Y, X)} is not a multiple of patch {(pz, py, px)}")
+    taps = [[float(t) for t in tt] for tt in (taps_y, taps_x)]
+    if not all(1 <= len(t) <= 16 for t in taps):
+        raise ValueError(f"{name}: 1 to 16 taps per axis, got {[len(t) for t in taps]}")
+    tabs = _state_tables(name, dev, C, mean=mean, std=std)
+    src = state.contiguous()
+    if px in (1, 2, 4) and X % 4 == 0 and src.data_ptr() % 16 == 0:
+        out = torch.empty((B, Z // pz, Y // py, X // px, C * pz * py * px), dtype=torch.bfloat16, device=dev)
+        if out.numel() == 0:
+            return out
+        a = _lib.StatePatchifyArgs()
+        a.state, a.tokens = src.data_ptr(), out.data_ptr()
+        a.mean = tabs["mean"].data_ptr() if tabs["mean"] is not None else None
+        a.std = tabs["std"].data_ptr() if tabs["std"] is not None else None
+        a.batch, a.channels = B, C
+        a.grid[:] = [Z, Y, X]
+        a.patch[:] = [pz, py, px]
+        fy, fx = ((ctypes.c_float * len(t))(*t) for t in taps)
+        lib = _lib.load()
+        with torch.cuda.device(dev):
+            rc = lib.strata_hip_dealias_patchify(ctypes.byref(a), fy, len(taps[0]), fx, len(taps[1]),
+                                                 ctypes.c_void_p(_stream(state)))
+        if rc == _lib.OK:
+            return out
+        if rc != _lib.EUNSUPPORTED:  # a patch too large for one workgroup's LDS takes the chain
+            raise _lib.StrataHipError("strata_hip_dealias_patchify", rc, lib.strata_hip_last_error().decode())
+    x, m, sd = src, tabs["mean"], tabs["std"]
+    for axis, p, t in ((1, py, taps[0]), (2, px, taps[1])):
+        if len(t) > 1:
+            x, m, sd = dealias_axis(x, m, sd, axis, p, t), None, None
+    return state_patchify(x, m, sd, (pz, py, px))
+
+
+@dealias_patchify.register_fake
+def _(state, mean, std, patch, taps_y, taps_x):
+    pz, py, px = _triple("patch", patch)
+    B, C, Z, Y, X = state.shape
+    return state.new_empty((B, Z // pz, Y // py, X // px, C * pz * py * px), dtype=torch.bfloat16)
+
+
+dealias_patchify.register_autograd(_no_backward("strata_hip::dealias_patchify"))
 
 
 @torch.library.custom_op("strata_hip::state_update", mutates_args=())

@@ -82,7 +82,10 @@ class PatchEmbed3D(nn.Module):
         self.proj = nn.Conv3d(in_chans, embed_dim, kernel_size=p, stride=p, bias=True)
 
     def forward(self, state: Tensor, mean: Optional[Tensor] = None, std: Optional[Tensor] = None) -> Tensor:
-        tok = ops.state_patchify(state.float(), mean, std, self.patch_size)
+        return self.embed(ops.state_patchify(state.float(), mean, std, self.patch_size))
+
+    def embed(self, tok: Tensor) -> Tensor:
+        """The embedding of patchified tokens ``[..., in_chans * prod(patch)]``."""
         w = self.proj.weight.reshape(self.embed_dim, -1).to(torch.bfloat16)
         K = w.shape[1]
         if K % 8:  # the GEMM takes K in multiples of 8: zero columns change nothing
@@ -104,8 +107,8 @@ class DealiasedPatchEmbed3D(PatchEmbed3D):
 
     Both stages are linear and each axis filter sums to 1, so the embedding is
     the plain patch embedding of the state filtered per decimated axis
-    (``strata_hip::dealias_axis``, the input normalisation fused into the first
-    pass): the GEMM does the plain embedding's FLOPs instead of a stride-1
+    (``strata_hip::dealias_axis`` along z, ``strata_hip::dealias_patchify`` along y
+    and x, the input normalisation fused into the first pass): the GEMM does the plain embedding's FLOPs instead of a stride-1
     conv's ``pz*py*px`` times as many."""
 
     def __init__(self, depth: int, height: int, width: int, patch_size: Sequence[int] | int = 16, in_chans: int = 3,
@@ -127,9 +130,8 @@ class DealiasedPatchEmbed3D(PatchEmbed3D):
 
     def forward(self, state: Tensor, mean: Optional[Tensor] = None, std: Optional[Tensor] = None) -> Tensor:
         x = state.float()
-        for axis, (p, taps) in enumerate(zip(self.patch_size, self.axis_taps)):
-            if len(taps) == 1:  # an identity pass (patch 1, or a one-tap filter)
-                continue
-            x = ops.dealias_axis(x, mean, std, axis, p, taps)
+        if len(self.axis_taps[0]) > 1:  # else an identity pass (patch 1, or a one-tap filter)
+            x = ops.dealias_axis(x, mean, std, 0, self.patch_size[0], self.axis_taps[0])
             mean = std = None  # normalised by the first pass
-        return super().forward(x, mean, std)
+        # the y and x passes and the patchify in one launch
+        return self.embed(ops.dealias_patchify(x, mean, std, self.patch_size, *self.axis_taps[1:]))

@@ -178,3 +178,74 @@ def test_dealiased_embed_is_state_dict_compatible(gpu):
     x = torch.randn(1, 4, 2, 8, 8, generator=torch.Generator().manual_seed(13)).to(gpu)
     with torch.no_grad():
         assert torch.equal(deal.to(gpu)(x), plain.to(gpu)(x))
+
+
+# (B, C, grid, patch): quads of the state over one, several and a ragged last workgroup, odd
+# channel counts (2-byte token pieces), tokens of 1, 2 and 4 columns, more rows than one pass
+WIDE_CASES = [(1, 1, (1, 1, 4), (1, 1, 1)), (2, 7, (2, 3, 132), (1, 1, 1)), (1, 33, (2, 6, 140), (1, 2, 2)),
+              (1, 80, (4, 4, 72), (2, 2, 2)), (2, 19, (1, 8, 36), (1, 4, 4)), (1, 300, (1, 2, 20), (1, 1, 1))]
+
+
+@pytest.mark.parametrize("case", WIDE_CASES, ids=str)
+@pytest.mark.parametrize("offset", [0, 1], ids=["aligned", "unaligned"])
+def test_state_kernels_by_quads(gpu, case, offset):
+    """Patchify and update bit-exact at the wide kernels' edges; a state that is only 4-byte
+    aligned takes the element-wise kernels and gives the same bits; the update in place."""
+    B, C, grid, patch = case
+    x, _ = _state((B, C, *grid), 3, gpu)
+    buf = torch.empty(x.numel() + offset, device=gpu)
+    xg = buf[offset:].view(x.shape)
+    xg.copy_(x)
+    g = torch.Generator().manual_seed(4)
+    mean, std = torch.randn(C, generator=g), torch.rand(C, generator=g) + 0.5
+    got = ops.state_patchify(xg, mean.to(gpu), std.to(gpu), patch)
+    assert torch.equal(got.cpu(), O.state_patchify(x, mean, std, patch))
+    P = patch[0] * patch[1] * patch[2]
+    pred = torch.randn(B, *(n // p for n, p in zip(grid, patch)), C * P, generator=g).bfloat16()
+    src = torch.arange(C, dtype=torch.int32)
+    src[0] = -1
+    floor = torch.full((C,), float("nan"))
+    floor[C // 2] = 0.0
+    for order in (0, 1):
+        args = [t.to(gpu) for t in (mean, std, src, floor)]
+        ref = O.state_update(pred, x, mean, std, src.tolist(), floor, grid, patch, order)
+        nxt = ops.state_update(pred.to(gpu), xg, *args, grid, patch, order)
+        assert torch.equal(nxt.cpu().nan_to_num(7.0), ref.nan_to_num(7.0))
+        a = _lib.StateUpdateArgs()  # next aliases state
+        inp, pg = xg.clone() if offset == 0 else xg, pred.to(gpu)
+        keep = inp.clone()
+        a.pred, a.next, a.state = pg.data_ptr(), inp.data_ptr(), inp.data_ptr()
+        a.mean, a.std, a.src_channel, a.clamp_min = (t.data_ptr() for t in args)
+        a.batch, a.channels, a.state_channels, a.order = B, C, C, order
+        a.grid[:], a.patch[:] = grid, patch
+        _lib.call("strata_hip_state_update", a, torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(inp.nan_to_num(7.0), nxt.nan_to_num(7.0))
+        inp.copy_(keep)
+
+
+@pytest.mark.parametrize("case", [
+    (1, 3, (1, 2, 4), (1, 2, 2), (3, 3)),       # every tap clamped
+    (2, 5, (2, 6, 36), (1, 2, 2), (5, 5)),
+    (1, 37, (1, 10, 132), (1, 2, 2), (4, 5)),   # columns over two workgroups, ragged row runs
+    (1, 6, (2, 12, 40), (1, 4, 4), (5, 4)),
+    (1, 9, (4, 8, 264), (2, 2, 2), (16, 16)),
+    (1, 5, (1, 12, 16), (1, 4, 2), (1, 5)),     # one axis unfiltered
+    (1, 5, (1, 12, 16), (1, 2, 4), (3, 1)),
+    (1, 4, (1, 6, 12), (1, 3, 1), (5, 3)),      # a patch height that is no power of two
+    (1, 4, (1, 6, 18), (1, 2, 2), (5, 5)),      # the three-launch chain: rows not in quads
+], ids=str)
+@pytest.mark.parametrize("norm", [False, True])
+def test_dealias_patchify_equals_the_chain(gpu, case, norm):
+    """The fused pass bit for bit against dealias_axis along y, then x, then the patchify,
+    non-finite inputs included."""
+    B, C, grid, patch, ntaps = case
+    _, xg = _state((B, C, *grid), 5, gpu)
+    g = torch.Generator().manual_seed(6)
+    m, s = (torch.randn(C, generator=g).to(gpu), (torch.rand(C, generator=g) + 0.5).to(gpu)) if norm else (None, None)
+    taps = [torch.softmax(torch.randn(n, generator=g), 0).tolist() for n in ntaps]
+    got = ops.dealias_patchify(xg, m, s, patch, *taps)
+    x = xg
+    for axis, t in ((1, taps[0]), (2, taps[1])):
+        if len(t) > 1:
+            x, m, s = ops.dealias_axis(x, m, s, axis, patch[axis], t), None, None
+    assert torch.equal(got, ops.state_patchify(x, m, s, patch))
