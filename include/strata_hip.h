@@ -325,6 +325,25 @@ typedef struct strata_hip_bias_grad_args {
 int64_t strata_hip_bias_grad_workspace(int64_t m, int64_t n);
 int strata_hip_bias_grad(const strata_hip_bias_grad_args* args, void* stream);
 
+/* ----------------------------------------------------------------------------
+ * Weight gradient of a Linear: out[n, k] = sum over m of g[m, n] * x[m, k], bf16
+ * in and out, fp32 accumulation in an order fixed by the shape.  n, k and the row
+ * strides multiples of 8, 16-byte aligned pointers.  workspace: fp32,
+ * strata_hip_weight_grad_workspace(m, n, k) elements (NULL when that is 0).
+ * ------------------------------------------------------------------------- */
+typedef struct strata_hip_weight_grad_args {
+  const void* g;
+  const void* x;
+  void* out; /* [n, k] contiguous */
+  float* workspace;
+  int64_t m, n, k;
+  int64_t ldg, ldx; /* row strides, elements */
+} strata_hip_weight_grad_args;
+
+int64_t strata_hip_weight_grad_workspace(int64_t m, int64_t n, int64_t k);
+int strata_hip_weight_grad(const strata_hip_weight_grad_args* args, void* stream);
+
+
 /* ---------------------------------------------------------------------------
  * Non-affine LayerNorm over the last dimension (the block's two pre-norms,
  * which carry no parameters in the state-dict manifests

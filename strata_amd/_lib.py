@@ -108,6 +108,20 @@ class GemmArgs(ctypes.Structure):
     ]
 
 
+class WeightGradArgs(ctypes.Structure):
+    _fields_ = [
+        ("g", ctypes.c_void_p),
+        ("x", ctypes.c_void_p),
+        ("out", ctypes.c_void_p),
+        ("workspace", ctypes.c_void_p),
+        ("m", ctypes.c_int64),
+        ("n", ctypes.c_int64),
+        ("k", ctypes.c_int64),
+        ("ldg", ctypes.c_int64),
+        ("ldx", ctypes.c_int64),
+    ]
+
+
 class LayerNormArgs(ctypes.Structure):
     _fields_ = [
         ("x", ctypes.c_void_p),
@@ -334,6 +348,8 @@ EXPORTS = {
     "strata_hip_cube_pad_faces": ([ctypes.POINTER(CubePadArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_cube_crop": ([ctypes.POINTER(CubeCropArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_state_patchify": ([ctypes.POINTER(StatePatchifyArgs), ctypes.c_void_p], ctypes.c_int),
+    "strata_hip_weight_grad": ([ctypes.POINTER(WeightGradArgs), ctypes.c_void_p], ctypes.c_int),
+    "strata_hip_weight_grad_workspace": ([ctypes.c_int64] * 3, ctypes.c_int64),
     "strata_hip_dealias_axis": ([ctypes.POINTER(DealiasAxisArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_dealias_patchify": (
         [ctypes.POINTER(StatePatchifyArgs), ctypes.POINTER(ctypes.c_float), ctypes.c_int32,

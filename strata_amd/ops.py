@@ -30,6 +30,7 @@ __all__ = [
     "gemm_bias_act",
     "gemm_gelu_train",
     "bias_grad",
+    "weight_grad",
     "layer_norm",
     "cube_pad_faces",
     "cube_crop",
@@ -639,7 +640,7 @@ def _gemm_backward(ctx, dout):
     g2 = g.reshape(-1, g.shape[-1])
     x2 = x.reshape(-1, x.shape[-1])
     dx = (g2 @ w).reshape(x.shape) if ctx.needs_input_grad[0] else None
-    dw = (g2.t() @ x2) if ctx.needs_input_grad[1] else None
+    dw = _linear_dw(g2, x2) if ctx.needs_input_grad[1] else None
     db = None
     if ctx.has_bias and ctx.needs_input_grad[2]:
         db = bias_grad(g2) if g2.shape[-1] % 8 == 0 else g2.float().sum(0).to(bias.dtype)
@@ -723,7 +724,7 @@ def _gelu_train_backward(ctx, dout, _ddact):
     g2 = (dact * dout).reshape(-1, dact.shape[-1])  # the gradient at the pre-activation
     x2 = x.reshape(-1, x.shape[-1])
     dx = (g2 @ w).reshape(x.shape) if ctx.needs_input_grad[0] else None
-    dw = (g2.t() @ x2) if ctx.needs_input_grad[1] else None
+    dw = _linear_dw(g2, x2) if ctx.needs_input_grad[1] else None
     db = None
     if ctx.has_bias and ctx.needs_input_grad[2]:
         db = bias_grad(g2) if g2.shape[-1] % 8 == 0 else g2.float().sum(0).to(torch.bfloat16)
@@ -763,6 +764,59 @@ def _(g):
 
 
 bias_grad.register_autograd(_no_backward("strata_hip::bias_grad"))
+
+
+@torch.library.custom_op("strata_hip::weight_grad", mutates_args=())
+def weight_grad(g: Tensor, x: Tensor) -> Tensor:
+    """``g.T @ x`` of ``g`` ``[M, N]`` and ``x`` ``[M, K]`` bf16 (fp32 accumulation in an order
+    fixed by the shape, rounded once to bf16): the weight gradient ``[N, K]`` of a Linear whose
+    output gradient is ``g`` and input ``x``.  N and K must be multiples of 8."""
+    name = "weight_grad"
+    _require_gpu(name, g, x)
+    if g.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or g.dim() != 2 or x.dim() != 2 or g.shape[0] != x.shape[0]:
+        raise ValueError(f"{name}: expected bfloat16 [M, N] and [M, K], got {g.dtype} {tuple(g.shape)}, "
+                         f"{x.dtype} {tuple(x.shape)}")
+    g2, x2 = _rows(name, g, "g"), _rows(name, x, "x")
+    (M, N), K = g2.shape, x2.shape[1]
+    if M == 0:
+        return g.new_zeros((N, K))
+    out = torch.empty((N, K), dtype=torch.bfloat16, device=g.device)
+    if out.numel() == 0:
+        return out
+    lib = _lib.load()
+    nws = int(lib.strata_hip_weight_grad_workspace(M, N, K))
+    ws = torch.empty(nws, dtype=torch.float32, device=g.device) if nws else None
+    a = _lib.WeightGradArgs()
+    a.g, a.x, a.out = g2.data_ptr(), x2.data_ptr(), out.data_ptr()
+    a.workspace = ws.data_ptr() if ws is not None else None
+    a.m, a.n, a.k = M, N, K
+    a.ldg, a.ldx = (g2.stride(0), x2.stride(0)) if M > 1 else (N, K)
+    with torch.cuda.device(g.device):
+        _lib.call("strata_hip_weight_grad", a, _stream(g))
+    return out
+
+
+@weight_grad.register_fake
+def _(g, x):
+    return g.new_empty((g.shape[1], x.shape[1]))
+
+
+def _weight_grad_setup_context(ctx, inputs, output):
+    ctx.save_for_backward(*inputs)
+
+
+def _weight_grad_backward(ctx, d):
+    """A second derivative (``create_graph``) through a Linear's weight gradient."""
+    g, x = ctx.saved_tensors
+    return (x @ d.t() if ctx.needs_input_grad[0] else None), (g @ d if ctx.needs_input_grad[1] else None)
+
+
+weight_grad.register_autograd(_weight_grad_backward, setup_context=_weight_grad_setup_context)
+
+
+def _linear_dw(g2: Tensor, x2: Tensor) -> Tensor:
+    """Weight gradient of a Linear: the HIP kernel, or torch's product for widths it does not take."""
+    return weight_grad(g2, x2) if g2.shape[1] % 8 == 0 and x2.shape[1] % 8 == 0 else g2.t() @ x2
 
 
 # ---------------------------------------------------------------------------

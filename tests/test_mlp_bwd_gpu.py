@@ -104,3 +104,33 @@ def test_gate_autograd_vs_torch(gpu, shape):
     (torch.sigmoid(F.linear(ref[0], ref[1], ref[2])) * ref[3]).backward(dout.float())
     for name, got, want in zip("xwba", leaves, ref):
         assert rel_l2(got.grad.float().cpu(), want.grad) <= 1e-2, name
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 8), (63, 64, 72), (64, 256, 256), (65, 264, 248), (257, 8, 520),
+                                   (1000, 384, 640), (20000, 200, 72), (70000, 264, 264)], ids=str)
+def test_weight_grad(gpu, shape):
+    """g.T @ x at the edges of a 64-row stage, a 256-column tile and a row split, against float64
+    (rounded once to bf16: 2^-9 of a value, 1.7e-3 of the norm; 3e-3 with the fp32 sums), from
+    rows of wider tensors too, and bit for bit on a repeat."""
+    M, N, K = shape
+    g = torch.Generator().manual_seed(M + N + K)
+    a, x = _bf((M, N + 8), g).to(gpu), _bf((M, K + 16), g).to(gpu)
+    ref = a[:, :N].double().t() @ x[:, 16:].double()
+    got = ops.weight_grad(a[:, :N], x[:, 16:])
+    assert rel_l2(got.float().cpu(), ref.float().cpu()) <= 3e-3
+    assert torch.equal(got, ops.weight_grad(a[:, :N].contiguous(), x[:, 16:].contiguous()))
+
+
+def test_weight_grad_second_derivative(gpu):
+    """create_graph through a Linear's weight gradient, against torch's own."""
+    g = torch.Generator().manual_seed(5)
+    x, w, v = _bf((40, 24), g), _bf((16, 24), g), _bf((16, 24), g)
+
+    def second(linear, dt):
+        xi, wi = (t.to(gpu, dt).requires_grad_(True) for t in (x, w))
+        (dw,) = torch.autograd.grad(linear(xi, wi).square().sum(), wi, create_graph=True)
+        return torch.autograd.grad((dw * v.to(gpu, dt)).sum(), xi)[0]
+
+    got = second(lambda a, b: ops.gemm_bias_act(a, b, None, None, _lib.ACT_NONE), torch.bfloat16)
+    ref = second(lambda a, b: F.linear(a, b), torch.float64)
+    assert rel_l2(got.double().cpu(), ref.cpu()) <= 2e-2
