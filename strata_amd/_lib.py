@@ -401,11 +401,20 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+def function(name: str):
+    """The library's function ``name`` (loaded once; argument and result types set)."""
+    return getattr(_lib if _lib is not None else load(), name)
+
+
+def raise_error(name: str, rc: int) -> None:
+    """The exception of a failed call: ``ValueError`` for invalid arguments."""
+    msg = load().strata_hip_last_error().decode(errors="replace")
+    if rc == EINVAL:
+        raise ValueError(f"{name}: {msg}")
+    raise StrataHipError(name, rc, msg)
+
+
 def call(name: str, args: ctypes.Structure, stream: int) -> None:
-    lib = load()
-    rc = getattr(lib, name)(ctypes.byref(args), ctypes.c_void_p(stream))
+    rc = function(name)(ctypes.byref(args), ctypes.c_void_p(stream))
     if rc != OK:
-        msg = lib.strata_hip_last_error().decode(errors="replace")
-        if rc == EINVAL:
-            raise ValueError(f"{name}: {msg}")
-        raise StrataHipError(name, rc, msg)
+        raise_error(name, rc)

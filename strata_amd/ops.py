@@ -44,22 +44,34 @@ __all__ = [
 ]
 
 
-def _stream(t: Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+def _launch(name: str, args: ctypes.Structure, t: Tensor, *extra) -> None:
+    """Enqueue the library's ``name(args, *extra, stream)`` on ``t``'s device and torch's
+    current stream there.  The small calls are bound by this host path, so it takes the
+    raw stream handle and changes the device only where it is another one (a
+    ``torch.cuda.Stream`` object and a device guard per launch cost 3.5 us of 21)."""
+    dev = t.get_device()
+    if dev == torch._C._cuda_getDevice():
+        rc = _lib.function(name)(ctypes.byref(args), *extra, torch._C._cuda_getCurrentRawStream(dev))
+    else:
+        with torch.cuda.device(dev):
+            rc = _lib.function(name)(ctypes.byref(args), *extra, torch._C._cuda_getCurrentRawStream(dev))
+    if rc != _lib.OK:
+        _lib.raise_error(name, rc)
 
 
-def _require_gpu(name: str, *ts: Optional[Tensor]) -> torch.device:
-    dev = None
+def _require_gpu(name: str, *ts: Optional[Tensor]) -> Optional[torch.device]:
+    first, dev = None, -1
     for t in ts:
         if t is None:
             continue
-        if not t.is_cuda:
+        d = t.get_device() if t.is_cuda else -1
+        if d < 0:
             raise ValueError(f"{name}: expected GPU tensors, got a tensor on {t.device}")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"{name}: tensors on different devices ({dev} and {t.device})")
-    return dev
+        if first is None:
+            first, dev = t, d
+        elif d != dev:
+            raise ValueError(f"{name}: tensors on different devices ({first.device} and {t.device})")
+    return first.device if first is not None else None
 
 
 def _dtype_code(name: str, t: Tensor) -> int:
@@ -82,9 +94,10 @@ def _triple(name: str, v: Sequence[int] | int) -> list[int]:
 def _token_strides(name: str, t: Tensor) -> list[int]:
     if t.dim() != 6:
         raise ValueError(f"{name}: expected a heads-last [B, Z, Y, X, H, D] tensor, got shape {tuple(t.shape)}")
-    if t.stride(-1) != 1:
+    st = t.stride()
+    if st[5] != 1:
         raise ValueError(f"{name}: the head_dim axis must be contiguous (stride 1)")
-    return [t.stride(i) for i in range(5)]
+    return list(st[:5])
 
 
 def _no_backward(op_name: str):
@@ -137,29 +150,16 @@ def _na3d_launch(name, q, k, v, kernel, dilation, scale, q_origin, q_extent, lse
         return out
     a = _na3d_args(q, k, v, out, dt, qs, ks, vs, kernel, dilation, scale, q_origin, q_extent)
     a.lse = lse.data_ptr() if lse is not None else None
-    with torch.cuda.device(q.device):
-        _lib.call("strata_hip_na3d_fwd", a, _stream(q))
+    _launch("strata_hip_na3d_fwd", a, q)
     return out
 
 
 def _na3d_args(q, k, v, out, dt, qs, ks, vs, kernel, dilation, scale, q_origin, q_extent) -> "_lib.Na3dArgs":
     B, Z, Y, X, H, D = q.shape
-    a = _lib.Na3dArgs()
-    a.q, a.k, a.v, a.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    a.dtype = dt
-    a.batch, a.heads, a.head_dim = B, H, D
-    a.grid[:] = [Z, Y, X]
-    a.q_origin[:] = q_origin
-    a.q_extent[:] = q_extent
-    a.kernel[:] = kernel
-    a.dilation[:] = dilation
-    a.scale = float(D**-0.5 if scale is None else scale)
-    a.q_stride[:] = qs
-    a.k_stride[:] = ks
-    a.v_stride[:] = vs
-    a.o_stride[:] = [out.stride(i) for i in range(5)]
-    a.lse = None
-    return a
+    return _lib.Na3dArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dt, B, H, D, (Z, Y, X),
+                         tuple(q_origin), tuple(q_extent), tuple(kernel), tuple(dilation), 0,
+                         float(D**-0.5 if scale is None else scale), 0.0, tuple(qs), tuple(ks), tuple(vs),
+                         out.stride()[:5], None)
 
 
 def _rope_q_tables(name, q, cos, sin):
@@ -221,14 +221,7 @@ def na3d_fwd_rope_q(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor, k
     if out.numel() == 0:
         return out
     a = _na3d_args(q, k, v, out, _dtype_code(name, q), qs, ks, vs, kernel, dilation, scale, [0, 0, 0], [Z, Y, X])
-    lib = _lib.load()
-    with torch.cuda.device(q.device):
-        rc = lib.strata_hip_na3d_fwd_rope_q(ctypes.byref(a), cos_c.data_ptr(), sin_c.data_ptr(), zt,
-                                            ctypes.c_void_p(_stream(q)))
-    if rc != _lib.OK:
-        msg = lib.strata_hip_last_error().decode(errors="replace")
-        raise (ValueError if rc == _lib.EINVAL else _lib.StrataHipError)(
-            *((f"{name}: {msg}",) if rc == _lib.EINVAL else ("strata_hip_na3d_fwd_rope_q", rc, msg)))
+    _launch("strata_hip_na3d_fwd_rope_q", a, q, cos_c.data_ptr(), sin_c.data_ptr(), zt)
     return out
 
 
@@ -308,8 +301,7 @@ def na3d_bwd(
             raise ValueError(f"{name}: lse must be float32 {tuple(shape[:5])} on {q.device}")
         lse = lse.contiguous()
         a.lse = lse.data_ptr()
-    with torch.cuda.device(q.device):
-        _lib.call("strata_hip_na3d_bwd", a, _stream(q))
+    _launch("strata_hip_na3d_bwd", a, q)
     return dq, dk, dv
 
 
@@ -424,20 +416,12 @@ def rope_qkv_pack(qkv: Tensor, cos: Tensor, sin: Tensor, heads: int, rope_layout
     v = torch.empty_like(k) if pack_v else k.new_empty(0)
     if k.numel() == 0:
         return q, k, v
-    a = _lib.RopePackArgs()
-    a.qkv, a.cos, a.sin = flat.data_ptr(), cos_c.data_ptr(), sin_c.data_ptr()
-    a.q, a.k, a.v = (q.data_ptr() if pack_q else None), k.data_ptr(), (v.data_ptr() if pack_v else None)
-    a.batch = B
-    a.grid[:] = [Z, Y, X]
-    a.table_z = cos.shape[1]
-    a.heads, a.head_dim, a.layout = heads, D, int(rope_layout)
-    a.qkv_row_stride = flat.stride(0)
-    a.qk_norm = 1 if qk_norm else 0
-    a.qk_norm_eps = float(qk_norm_eps)
-    a.q_norm_weight = wts[0].data_ptr() if wts[0] is not None else None
-    a.k_norm_weight = wts[1].data_ptr() if wts[1] is not None else None
-    with torch.cuda.device(qkv.device):
-        _lib.call("strata_hip_rope_qkv_pack", a, _stream(qkv))
+    a = _lib.RopePackArgs(flat.data_ptr(), cos_c.data_ptr(), sin_c.data_ptr(), q.data_ptr() if pack_q else None,
+                          k.data_ptr(), v.data_ptr() if pack_v else None, B, (Z, Y, X), cos.shape[1], heads, D,
+                          int(rope_layout), flat.stride(0), 1 if qk_norm else 0, float(qk_norm_eps),
+                          wts[0].data_ptr() if wts[0] is not None else None,
+                          wts[1].data_ptr() if wts[1] is not None else None)
+    _launch("strata_hip_rope_qkv_pack", a, qkv)
     return q, k, v
 
 
@@ -499,8 +483,7 @@ def _rope_backward(ctx, dq, dk, dv):
         a.dq_norm_weight = dws[0].data_ptr() if dws[0] is not None else None
         a.dk_norm_weight = dws[1].data_ptr() if dws[1] is not None else None
     if dqkv.numel():
-        with torch.cuda.device(cos.device):
-            _lib.call("strata_hip_rope_qkv_pack_bwd", a, _stream(dqkv))
+        _launch("strata_hip_rope_qkv_pack_bwd", a, dqkv)
     if ctx.qk_norm:
         dws = [d.to(w.dtype) if d is not None else None for d, w in zip(dws, ctx.saved_tensors[3:])]
     return dqkv, None, None, None, None, None, None, dws[0], dws[1], None, None
@@ -521,6 +504,18 @@ def _rows(name: str, t: Tensor, what: str) -> Tensor:
     if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) % 8) or t2.data_ptr() % 16:
         t2 = t2.contiguous()
     return t2
+
+
+def _row_view(t: Tensor, cols: int) -> tuple[int, int, int, Tensor]:
+    """Rows, data pointer and row stride of t as a [rows, cols] matrix, and the tensor that
+    holds them (t, or the copy ``_rows`` makes where t's layout needs one)."""
+    if t.is_contiguous():
+        ptr = t.data_ptr()
+        if ptr % 16 == 0 and cols % 8 == 0 and cols:
+            return t.numel() // cols, ptr, cols, t
+    t2 = _rows("", t, "")
+    rows = t2.shape[0]
+    return rows, t2.data_ptr(), t2.stride(0) if rows > 1 else cols, t2
 
 
 def _pad_n(w: Tensor, bias: Optional[Tensor], residual: Optional[Tensor]):
@@ -577,30 +572,20 @@ def gemm_bias_act(x: Tensor, w: Tensor, bias: Optional[Tensor], residual: Option
 def _gemm_launch(x: Tensor, w: Tensor, bias: Optional[Tensor], residual: Optional[Tensor], act: int,
                  res_op: int) -> Tensor:
     """strata_hip_gemm_bias_act on validated operands whose N is a multiple of 8."""
-    name = "gemm_bias_act"
     K, N = x.shape[-1], w.shape[0]
     out_shape = (*x.shape[:-1], N)
-    x2 = _rows(name, x, "x")
-    w2 = _rows(name, w, "w")
+    M, xp, ldx, x2 = _row_view(x, K)
+    _, wp, ldw, w2 = _row_view(w, K)
     b2 = bias.contiguous() if bias is not None else None
-    r2 = _rows(name, residual, "residual") if residual is not None else None
+    rp, ldr, r2 = None, 0, None
+    if residual is not None:
+        _, rp, ldr, r2 = _row_view(residual, N)
     out = torch.empty(out_shape, dtype=torch.bfloat16, device=x.device)
-    M = x2.shape[0]
     if M == 0 or N == 0:
         return out
-    a = _lib.GemmArgs()
-    a.x, a.w = x2.data_ptr(), w2.data_ptr()
-    a.bias = b2.data_ptr() if b2 is not None else None
-    a.residual = r2.data_ptr() if r2 is not None else None
-    a.out = out.data_ptr()
-    a.m, a.n, a.k = M, N, K
-    a.ldx, a.ldw = x2.stride(0) if M > 1 else K, w2.stride(0) if N > 1 else K
-    a.ldr = (r2.stride(0) if M > 1 else N) if r2 is not None else 0
-    a.ldo = N
-    a.act = int(act)
-    a.res_op = int(res_op)
-    with torch.cuda.device(x.device):
-        _lib.call("strata_hip_gemm_bias_act", a, _stream(x))
+    a = _lib.GemmArgs(xp, wp, b2.data_ptr() if b2 is not None else None, rp, out.data_ptr(), M, N, K, ldx, ldw, ldr, N,
+                      int(act), int(res_op))
+    _launch("strata_hip_gemm_bias_act", a, x)
     return out
 
 
@@ -696,12 +681,7 @@ def _gemm_gelu_train_launch(x: Tensor, w: Tensor, bias: Optional[Tensor]) -> tup
     a.ldx, a.ldw = x2.stride(0) if M > 1 else K, w2.stride(0) if N > 1 else K
     a.ldr, a.ldo = 0, N
     a.act, a.res_op = _lib.ACT_GELU_TANH, _lib.RES_ADD
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        rc = lib.strata_hip_gemm_gelu_save(ctypes.byref(a), ctypes.c_void_p(dact.data_ptr()),
-                                           ctypes.c_void_p(_stream(x)))
-    if rc != _lib.OK:
-        raise _lib.StrataHipError("strata_hip_gemm_gelu_save", rc, lib.strata_hip_last_error().decode())
+    _launch("strata_hip_gemm_gelu_save", a, x, dact.data_ptr())
     return out, dact
 
 
@@ -753,8 +733,7 @@ def bias_grad(g: Tensor) -> Tensor:
     a = _lib.BiasGradArgs()
     a.g, a.out, a.workspace = g2.data_ptr(), out.data_ptr(), ws.data_ptr()
     a.m, a.n, a.ldg = M, N, (g2.stride(0) if M > 1 else N)
-    with torch.cuda.device(g.device):
-        _lib.call("strata_hip_bias_grad", a, _stream(g))
+    _launch("strata_hip_bias_grad", a, g)
     return out
 
 
@@ -791,8 +770,7 @@ def weight_grad(g: Tensor, x: Tensor) -> Tensor:
     a.workspace = ws.data_ptr() if ws is not None else None
     a.m, a.n, a.k = M, N, K
     a.ldg, a.ldx = (g2.stride(0), x2.stride(0)) if M > 1 else (N, K)
-    with torch.cuda.device(g.device):
-        _lib.call("strata_hip_weight_grad", a, _stream(g))
+    _launch("strata_hip_weight_grad", a, g)
     return out
 
 
@@ -829,18 +807,13 @@ def layer_norm(x: Tensor, eps: float) -> Tensor:
     _require_gpu(name, x)
     if x.dtype != torch.bfloat16:
         raise ValueError(f"{name}: x must be bfloat16")
-    x2 = _rows(name, x, "x")
+    C = x.shape[-1]
+    M, xp, ldx, x2 = _row_view(x, C)
     out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    if x2.shape[0] == 0:
+    if M == 0:
         return out
-    a = _lib.LayerNormArgs()
-    a.x, a.out = x2.data_ptr(), out.data_ptr()
-    a.m, a.c = x2.shape[0], x2.shape[1]
-    a.ldx = x2.stride(0) if x2.shape[0] > 1 else x2.shape[1]
-    a.ldo = x2.shape[1]
-    a.eps = float(eps)
-    with torch.cuda.device(x.device):
-        _lib.call("strata_hip_layer_norm", a, _stream(x))
+    a = _lib.LayerNormArgs(xp, out.data_ptr(), M, C, ldx, C, float(eps))
+    _launch("strata_hip_layer_norm", a, x)
     return out
 
 
@@ -864,8 +837,7 @@ def _ln_backward(ctx, dy):
         a = _lib.LayerNormBwdArgs()
         a.x, a.dy, a.dx = x2.data_ptr(), g2.data_ptr(), dx.data_ptr()
         a.m, a.c, a.ld, a.eps = x2.shape[0], x2.shape[1], x2.shape[1], ctx.eps
-        with torch.cuda.device(x.device):
-            _lib.call("strata_hip_layer_norm_bwd", a, _stream(x))
+        _launch("strata_hip_layer_norm_bwd", a, x)
     return dx.view(x.shape), None
 
 
@@ -905,8 +877,7 @@ def cube_pad_faces(data: Tensor, pad: int) -> Tensor:
     a.src, a.dst = src.data_ptr(), out.data_ptr()
     a.dtype, a.face_size, a.pad = _CUBE_DTYPES[data.dtype], n, int(pad)
     a.lead = src.numel() // (6 * n * n)
-    with torch.cuda.device(data.device):
-        _lib.call("strata_hip_cube_pad_faces", a, _stream(data))
+    _launch("strata_hip_cube_pad_faces", a, data)
     return out
 
 
@@ -940,8 +911,7 @@ def cube_crop(x: Tensor, halo: int) -> Tensor:
     a.src, a.dst = src.data_ptr(), out.data_ptr()
     a.dtype, a.extent, a.halo = _CUBE_DTYPES[x.dtype], S, int(halo)
     a.planes = src.numel() // (S * S)
-    with torch.cuda.device(x.device):
-        _lib.call("strata_hip_cube_crop", a, _stream(x))
+    _launch("strata_hip_cube_crop", a, x)
     return out
 
 
@@ -1002,8 +972,7 @@ def state_patchify(
     a.batch, a.channels = B, C
     a.grid[:] = [Z, Y, X]
     a.patch[:] = [pz, py, px]
-    with torch.cuda.device(dev):
-        _lib.call("strata_hip_state_patchify", a, _stream(state))
+    _launch("strata_hip_state_patchify", a, state)
     return out
 
 
@@ -1053,8 +1022,7 @@ def dealias_axis(
     a.grid[:] = [Z, Y, X]
     a.axis, a.patch, a.taps = axis, patch, len(taps)
     a.filter[: len(taps)] = taps
-    with torch.cuda.device(dev):
-        _lib.call("strata_hip_dealias_axis", a, _stream(state))
+    _launch("strata_hip_dealias_axis", a, state)
     return out
 
 
@@ -1101,14 +1069,12 @@ def dealias_patchify(
         a.grid[:] = [Z, Y, X]
         a.patch[:] = [pz, py, px]
         fy, fx = ((ctypes.c_float * len(t))(*t) for t in taps)
-        lib = _lib.load()
-        with torch.cuda.device(dev):
-            rc = lib.strata_hip_dealias_patchify(ctypes.byref(a), fy, len(taps[0]), fx, len(taps[1]),
-                                                 ctypes.c_void_p(_stream(state)))
-        if rc == _lib.OK:
+        try:
+            _launch("strata_hip_dealias_patchify", a, state, fy, len(taps[0]), fx, len(taps[1]))
             return out
-        if rc != _lib.EUNSUPPORTED:  # a patch too large for one workgroup's LDS takes the chain
-            raise _lib.StrataHipError("strata_hip_dealias_patchify", rc, lib.strata_hip_last_error().decode())
+        except _lib.StrataHipError as e:
+            if e.code != _lib.EUNSUPPORTED:  # a patch too large for one workgroup's LDS takes the chain
+                raise
     x, m, sd = src, tabs["mean"], tabs["std"]
     for axis, p, t in ((1, py, taps[0]), (2, px, taps[1])):
         if len(t) > 1:
@@ -1189,8 +1155,7 @@ def state_update(
     a.batch, a.channels, a.state_channels, a.order = B, C, Cin, int(order)
     a.grid[:] = [Z, Y, X]
     a.patch[:] = [pz, py, px]
-    with torch.cuda.device(dev):
-        _lib.call("strata_hip_state_update", a, _stream(pred))
+    _launch("strata_hip_state_update", a, pred)
     return out
 
 
@@ -1240,8 +1205,7 @@ def upsample_dw_gelu(cond: Tensor, weight: Tensor, bias: Optional[Tensor], facto
     a.batch, a.depth, a.height, a.width, a.channels, a.factor = B, Z, Yc, Xc, C, f
     a.cond_stride[:] = [c.stride(i) for i in range(4)]
     a.out_stride[:] = [out.stride(i) for i in range(4)]
-    with torch.cuda.device(cond.device):
-        _lib.call("strata_hip_upsample_dw_gelu", a, _stream(cond))
+    _launch("strata_hip_upsample_dw_gelu", a, cond)
     return out
 
 
@@ -1273,8 +1237,7 @@ def layer_norm_modulate(x: Tensor, shift: Tensor, scale: Tensor, eps: float) -> 
     ld = lambda t: t.stride(0) if t.shape[0] > 1 else t.shape[1]  # noqa: E731
     a.ldx, a.ldo, a.ld_shift, a.ld_scale = ld(x2), x2.shape[1], ld(sh), ld(sc)
     a.eps = float(eps)
-    with torch.cuda.device(x.device):
-        _lib.call("strata_hip_layer_norm_modulate", a, _stream(x))
+    _launch("strata_hip_layer_norm_modulate", a, x)
     return out
 
 
@@ -1303,8 +1266,7 @@ def gated_add(res: Tensor, gate: Tensor, y: Tensor) -> Tensor:
     a.m, a.c = r2.shape
     ld = lambda t: t.stride(0) if t.shape[0] > 1 else t.shape[1]  # noqa: E731
     a.ld_res, a.ld_gate, a.ld_y, a.ld_out = ld(r2), ld(g2), ld(y2), r2.shape[1]
-    with torch.cuda.device(res.device):
-        _lib.call("strata_hip_gated_add", a, _stream(res))
+    _launch("strata_hip_gated_add", a, res)
     return out
 
 
