@@ -327,9 +327,11 @@ int strata_hip_bias_grad(const strata_hip_bias_grad_args* args, void* stream);
 
 /* ----------------------------------------------------------------------------
  * Weight gradient of a Linear: out[n, k] = sum over m of g[m, n] * x[m, k], bf16
- * in and out, fp32 accumulation in an order fixed by the shape.  n, k and the row
- * strides multiples of 8, 16-byte aligned pointers.  workspace: fp32,
- * strata_hip_weight_grad_workspace(m, n, k) elements (NULL when that is 0).
+ * in and out, fp32 accumulation in an order fixed by the shape; with bias_out also
+ * the bias gradient bias_out[n] = sum over m of g[m, n].  n, k and the row strides
+ * multiples of 8, 16-byte aligned pointers (bias_out: 2-byte).  workspace: fp32,
+ * strata_hip_weight_grad_workspace(m, n, k, bias_out != NULL) elements (NULL when
+ * that is 0).
  * ------------------------------------------------------------------------- */
 typedef struct strata_hip_weight_grad_args {
   const void* g;
@@ -338,9 +340,10 @@ typedef struct strata_hip_weight_grad_args {
   float* workspace;
   int64_t m, n, k;
   int64_t ldg, ldx; /* row strides, elements */
+  void* bias_out;   /* [n] or NULL */
 } strata_hip_weight_grad_args;
 
-int64_t strata_hip_weight_grad_workspace(int64_t m, int64_t n, int64_t k);
+int64_t strata_hip_weight_grad_workspace(int64_t m, int64_t n, int64_t k, int32_t bias);
 int strata_hip_weight_grad(const strata_hip_weight_grad_args* args, void* stream);
 
 

@@ -119,6 +119,7 @@ class WeightGradArgs(ctypes.Structure):
         ("k", ctypes.c_int64),
         ("ldg", ctypes.c_int64),
         ("ldx", ctypes.c_int64),
+        ("bias_out", ctypes.c_void_p),
     ]
 
 
@@ -349,7 +350,7 @@ EXPORTS = {
     "strata_hip_cube_crop": ([ctypes.POINTER(CubeCropArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_state_patchify": ([ctypes.POINTER(StatePatchifyArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_weight_grad": ([ctypes.POINTER(WeightGradArgs), ctypes.c_void_p], ctypes.c_int),
-    "strata_hip_weight_grad_workspace": ([ctypes.c_int64] * 3, ctypes.c_int64),
+    "strata_hip_weight_grad_workspace": ([ctypes.c_int64] * 3 + [ctypes.c_int32], ctypes.c_int64),
     "strata_hip_dealias_axis": ([ctypes.POINTER(DealiasAxisArgs), ctypes.c_void_p], ctypes.c_int),
     "strata_hip_dealias_patchify": (
         [ctypes.POINTER(StatePatchifyArgs), ctypes.POINTER(ctypes.c_float), ctypes.c_int32,

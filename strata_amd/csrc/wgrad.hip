@@ -13,6 +13,12 @@
 // fp32 partial and a second launch adds the partials in split order: the order of
 // every addition is fixed by the shape, the result repeats bit for bit.
 //
+// With a bias gradient (the column sums of g) each of a row range's workgroups along
+// k sums its share of the stages, 4 more MFMAs beside 32 there (a ones operand
+// against the g fragments it holds anyway); the partials, [splits * kt, N] fp32, are
+// added in the second launch: at [65536, 3072] 11 us more here in the place of a 39 us
+// pass over g of its own.
+//
 // Bound by the copies and LDS reads beside the MFMAs, as the forward's 256 x 256
 // kernel (same tile, ring and burst split).  Against the library's product, us:
 // [65536, N] x [65536, K] of N x K = 3072 x 768 433 -> 292, 2304 x 768 526 -> 233,
@@ -26,6 +32,7 @@ struct WgradParams {
   const bf16* g;
   const bf16* x;
   float* part;  // [splits, N, K] fp32, or null: one split, straight to out
+  float* bpart; // [splits * kt, N] fp32 column sums of g, or null
   bf16* out;    // [N, K]
   int64_t M, N, K, ldg, ldx;
   int nt, kt;   // 256-wide tiles along N and K
@@ -36,6 +43,7 @@ constexpr int WG_BK = 64;                    // rows per stage
 constexpr int WG_HALF = WG_BK * 512;         // bytes of one panel's stage
 constexpr int WG_STAGE = 2 * WG_HALF;
 
+template <bool BIAS>
 __global__ __launch_bounds__(512, 1) void weight_grad_kernel(WgradParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NW = 8, LPW = WG_HALF / 1024 / NW;  // 1-KiB copies per wave, panel and stage
@@ -103,9 +111,18 @@ __global__ __launch_bounds__(512, 1) void weight_grad_kernel(WgradParams p) {
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  f32x4 bacc[BIAS ? 4 : 1];
+  bf16x8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = (bf16)1.f;
+#pragma unroll
+  for (int j = 0; j < (BIAS ? 4 : 1); ++j) bacc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int btick = tk;  // stages until this workgroup's next turn at the column sums
   issue(0, 0, false);
   issue(0, 0, true);
   for (int kt = 0; kt < nk; ++kt) {
+    const bool mine = BIAS && btick == 0 && wk == 0;  // uniform
+    if (BIAS) btick = btick == 0 ? p.kt - 1 : btick - 1;
     wait_vmcnt(0);
     lds_barrier();  // the stage has landed for every wave; the other slot is free
     const int wr = (kt + 1) & 1;
@@ -123,15 +140,30 @@ __global__ __launch_bounds__(512, 1) void weight_grad_kernel(WgradParams p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      if constexpr (BIAS) {
+        if (mine) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bacc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[j], bacc[j], 0, 0, 0);
+        }
+      }
       if (kk == 0 && kt + 1 < nk) {
         __builtin_amdgcn_sched_barrier(0);
         issue(kt + 1, wr, true);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    __builtin_amdgcn_iglp_opt(1);
+    if constexpr (!BIAS) __builtin_amdgcn_iglp_opt(1);
   }
 
+  if constexpr (BIAS) {
+    if (wk == 0 && g4 == 0) {  // every row of the ones product holds the sums
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t n = n0 + 64 * wn + 16 * j + n16;
+        if (n < p.N) p.bpart[((int64_t)sp * p.kt + tk) * p.N + n] = bacc[j][0];
+      }
+    }
+  }
   // Block (i, j): k = 128 wk + 16 i + 4 g4 + r, n = 64 wn + 16 j + n16.  N and K are
   // multiples of 8: a quad lies inside the matrix or outside it.
 #pragma unroll
@@ -153,9 +185,28 @@ __global__ __launch_bounds__(512, 1) void weight_grad_kernel(WgradParams p) {
 #endif
 }
 
-// out = the sum of the partials in split order, eight elements per thread.
+// out = the sum of the partials in split order, eight elements per thread; the last
+// blocks the bias gradient's, 16 columns each, 16 threads a column: each adds every
+// 16th partial in order, then the 16 sums in order.
 __global__ __launch_bounds__(256) void weight_grad_finish_kernel(const float* __restrict__ part, bf16* __restrict__ out,
-                                                                 int64_t n, int splits) {
+                                                                 int64_t n, int splits, int blocks,
+                                                                 const float* __restrict__ bpart,
+                                                                 bf16* __restrict__ bout, int64_t N, int bsplits) {
+  if ((int)blockIdx.x >= blocks) {
+    __shared__ float red[16][16];
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+    const int64_t col = ((int64_t)blockIdx.x - blocks) * 16 + c;
+    float s = 0.f;
+    if (col < N)
+      for (int k = r; k < bsplits; k += 16) s += bpart[(int64_t)k * N + col];
+    red[r][c] = s;
+    __syncthreads();
+    if (r == 0 && col < N) {
+      for (int k = 1; k < 16; ++k) s += red[k][c];
+      bout[col] = (bf16)s;
+    }
+    return;
+  }
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
   if (i >= n) return;
   f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
@@ -178,12 +229,17 @@ static int wgrad_splits(int64_t m, int64_t n, int64_t k) {
   return (int)(s < most ? s : most);
 }
 
+// fp32 elements of the bias partials, a multiple of 4 (the weight partials follow).
+static int64_t wgrad_bias_floats(int64_t n, int64_t k, int64_t splits) {
+  return (splits * ((k + 255) / 256) * n + 3) / 4 * 4;
+}
+
 }  // namespace strata
 
-extern "C" int64_t strata_hip_weight_grad_workspace(int64_t m, int64_t n, int64_t k) {
+extern "C" int64_t strata_hip_weight_grad_workspace(int64_t m, int64_t n, int64_t k, int32_t bias) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   const int64_t s = strata::wgrad_splits(m, n, k);
-  return s > 1 ? s * n * k : 0;
+  return (s > 1 ? s * n * k : 0) + (bias ? strata::wgrad_bias_floats(n, k, s) : 0);
 }
 
 extern "C" int strata_hip_weight_grad(const strata_hip_weight_grad_args* a, void* stream) {
@@ -215,16 +271,20 @@ extern "C" int strata_hip_weight_grad(const strata_hip_weight_grad_args* a, void
     return fail(STRATA_HIP_EUNSUPPORTED, "weight_grad: problem too large for one launch");
   p.rows = (int)(per * WG_BK);
   p.splits = (int)((stages + per - 1) / per);  // ranges that hold rows
-  if (want > 1) {
+  const bool bias = a->bias_out != nullptr;
+  if (want > 1 || bias) {
     if (!a->workspace) return fail(STRATA_HIP_EINVAL, "weight_grad: null workspace");
-    p.part = a->workspace;
+    if (bias) p.bpart = a->workspace;
+    if (want > 1) p.part = a->workspace + (bias ? wgrad_bias_floats(a->n, a->k, want) : 0);
   }
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(weight_grad_kernel, dim3((unsigned)(p.nt * p.kt * p.splits)), dim3(512), 0, st, p);
-  if (p.part) {
-    const int64_t n = a->n * a->k;
-    hipLaunchKernelGGL(weight_grad_finish_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st, p.part, p.out,
-                       n, p.splits);
-  }
+  const dim3 grid((unsigned)(p.nt * p.kt * p.splits));
+  if (bias) hipLaunchKernelGGL(weight_grad_kernel<true>, grid, dim3(512), 0, st, p);
+  else hipLaunchKernelGGL(weight_grad_kernel<false>, grid, dim3(512), 0, st, p);
+  const int64_t n = a->n * a->k;
+  const int blocks = p.part ? (int)((n / 8 + 255) / 256) : 0, bblocks = bias ? (int)((a->n + 15) / 16) : 0;
+  if (blocks + bblocks)
+    hipLaunchKernelGGL(weight_grad_finish_kernel, dim3((unsigned)(blocks + bblocks)), dim3(256), 0, st, p.part, p.out, n,
+                       p.splits, blocks, p.bpart, (bf16*)a->bias_out, a->n, p.splits * p.kt);
   return check_launch("weight_grad kernels");
 }

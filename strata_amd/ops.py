@@ -30,7 +30,7 @@ __all__ = [
     "gemm_bias_act",
     "gemm_gelu_train",
     "bias_grad",
-    "weight_grad",
+    "linear_grads",
     "layer_norm",
     "cube_pad_faces",
     "cube_crop",
@@ -625,10 +625,7 @@ def _gemm_backward(ctx, dout):
     g2 = g.reshape(-1, g.shape[-1])
     x2 = x.reshape(-1, x.shape[-1])
     dx = (g2 @ w).reshape(x.shape) if ctx.needs_input_grad[0] else None
-    dw = _linear_dw(g2, x2) if ctx.needs_input_grad[1] else None
-    db = None
-    if ctx.has_bias and ctx.needs_input_grad[2]:
-        db = bias_grad(g2) if g2.shape[-1] % 8 == 0 else g2.float().sum(0).to(bias.dtype)
+    dw, db = _param_grads(ctx, g2, x2)
     if not gate:
         dres = dout if ctx.has_res and ctx.needs_input_grad[3] else None
     return dx, dw, db, dres, None, None
@@ -704,10 +701,7 @@ def _gelu_train_backward(ctx, dout, _ddact):
     g2 = (dact * dout).reshape(-1, dact.shape[-1])  # the gradient at the pre-activation
     x2 = x.reshape(-1, x.shape[-1])
     dx = (g2 @ w).reshape(x.shape) if ctx.needs_input_grad[0] else None
-    dw = _linear_dw(g2, x2) if ctx.needs_input_grad[1] else None
-    db = None
-    if ctx.has_bias and ctx.needs_input_grad[2]:
-        db = bias_grad(g2) if g2.shape[-1] % 8 == 0 else g2.float().sum(0).to(torch.bfloat16)
+    dw, db = _param_grads(ctx, g2, x2)
     return dx, dw, db
 
 
@@ -745,56 +739,71 @@ def _(g):
 bias_grad.register_autograd(_no_backward("strata_hip::bias_grad"))
 
 
-@torch.library.custom_op("strata_hip::weight_grad", mutates_args=())
-def weight_grad(g: Tensor, x: Tensor) -> Tensor:
-    """``g.T @ x`` of ``g`` ``[M, N]`` and ``x`` ``[M, K]`` bf16 (fp32 accumulation in an order
-    fixed by the shape, rounded once to bf16): the weight gradient ``[N, K]`` of a Linear whose
-    output gradient is ``g`` and input ``x``.  N and K must be multiples of 8."""
-    name = "weight_grad"
+@torch.library.custom_op("strata_hip::linear_grads", mutates_args=())
+def linear_grads(g: Tensor, x: Tensor, bias: bool) -> tuple[Tensor, Tensor]:
+    """Parameter gradients of a Linear with output gradient ``g`` ``[M, N]`` and input ``x``
+    ``[M, K]`` (bf16, fp32 accumulation in an order fixed by the shape, rounded once): the
+    weight's ``g.T @ x`` ``[N, K]`` and, with ``bias``, the bias's column sums of ``g`` ``[N]``
+    (else an empty tensor).  N and K must be multiples of 8."""
+    name = "linear_grads"
     _require_gpu(name, g, x)
     if g.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or g.dim() != 2 or x.dim() != 2 or g.shape[0] != x.shape[0]:
         raise ValueError(f"{name}: expected bfloat16 [M, N] and [M, K], got {g.dtype} {tuple(g.shape)}, "
                          f"{x.dtype} {tuple(x.shape)}")
     g2, x2 = _rows(name, g, "g"), _rows(name, x, "x")
     (M, N), K = g2.shape, x2.shape[1]
-    if M == 0:
-        return g.new_zeros((N, K))
+    if M == 0 or N == 0 or K == 0:
+        return g.new_zeros((N, K)), g.sum(0) if bias else g.new_empty(0)
     out = torch.empty((N, K), dtype=torch.bfloat16, device=g.device)
-    if out.numel() == 0:
-        return out
-    lib = _lib.load()
-    nws = int(lib.strata_hip_weight_grad_workspace(M, N, K))
+    db = torch.empty(N if bias else 0, dtype=torch.bfloat16, device=g.device)
+    nws = int(_lib.load().strata_hip_weight_grad_workspace(M, N, K, int(bias)))
     ws = torch.empty(nws, dtype=torch.float32, device=g.device) if nws else None
-    a = _lib.WeightGradArgs()
-    a.g, a.x, a.out = g2.data_ptr(), x2.data_ptr(), out.data_ptr()
-    a.workspace = ws.data_ptr() if ws is not None else None
-    a.m, a.n, a.k = M, N, K
-    a.ldg, a.ldx = (g2.stride(0), x2.stride(0)) if M > 1 else (N, K)
+    ldg, ldx = (g2.stride(0), x2.stride(0)) if M > 1 else (N, K)
+    a = _lib.WeightGradArgs(g2.data_ptr(), x2.data_ptr(), out.data_ptr(), ws.data_ptr() if ws is not None else None,
+                            M, N, K, ldg, ldx, db.data_ptr() if bias else None)
     _launch("strata_hip_weight_grad", a, g)
-    return out
+    return out, db
 
 
-@weight_grad.register_fake
-def _(g, x):
-    return g.new_empty((g.shape[1], x.shape[1]))
+@linear_grads.register_fake
+def _(g, x, bias):
+    return g.new_empty((g.shape[1], x.shape[1])), g.new_empty((g.shape[1] if bias else 0,))
 
 
-def _weight_grad_setup_context(ctx, inputs, output):
-    ctx.save_for_backward(*inputs)
+def _linear_grads_setup_context(ctx, inputs, output):
+    ctx.bias = inputs[2]
+    ctx.save_for_backward(*inputs[:2])
 
 
-def _weight_grad_backward(ctx, d):
-    """A second derivative (``create_graph``) through a Linear's weight gradient."""
+def _linear_grads_backward(ctx, d, db):
+    """A second derivative (``create_graph``) through a Linear's parameter gradients."""
     g, x = ctx.saved_tensors
-    return (x @ d.t() if ctx.needs_input_grad[0] else None), (g @ d if ctx.needs_input_grad[1] else None)
+    dg = dx = None
+    if ctx.needs_input_grad[0]:
+        dg = x @ d.t() if d is not None else torch.zeros_like(g)
+        if ctx.bias and db is not None:
+            dg = dg + db
+    if ctx.needs_input_grad[1] and d is not None:
+        dx = g @ d
+    return dg, dx, None
 
 
-weight_grad.register_autograd(_weight_grad_backward, setup_context=_weight_grad_setup_context)
+linear_grads.register_autograd(_linear_grads_backward, setup_context=_linear_grads_setup_context)
 
 
-def _linear_dw(g2: Tensor, x2: Tensor) -> Tensor:
-    """Weight gradient of a Linear: the HIP kernel, or torch's product for widths it does not take."""
-    return weight_grad(g2, x2) if g2.shape[1] % 8 == 0 and x2.shape[1] % 8 == 0 else g2.t() @ x2
+def _param_grads(ctx, g2: Tensor, x2: Tensor) -> tuple[Optional[Tensor], Optional[Tensor]]:
+    """The weight's and the bias's gradients a GEMM op's backward owes (inputs 1 and 2), each
+    None where none is wanted; torch's products for widths the kernel does not take."""
+    want_w, want_b = ctx.needs_input_grad[1], ctx.has_bias and ctx.needs_input_grad[2]
+    N, K = g2.shape[1], x2.shape[1]
+    if want_w and N % 8 == 0 and K % 8 == 0:
+        dw, db = linear_grads(g2, x2, want_b)
+        return dw, db if want_b else None
+    dw = g2.t() @ x2 if want_w else None
+    db = None
+    if want_b:
+        db = bias_grad(g2) if N % 8 == 0 else g2.float().sum(0).to(g2.dtype)
+    return dw, db
 
 
 # ---------------------------------------------------------------------------

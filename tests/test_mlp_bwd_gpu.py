@@ -108,20 +108,23 @@ def test_gate_autograd_vs_torch(gpu, shape):
 
 @pytest.mark.parametrize("shape", [(1, 8, 8), (63, 64, 72), (64, 256, 256), (65, 264, 248), (257, 8, 520),
                                    (1000, 384, 640), (20000, 200, 72), (70000, 264, 264)], ids=str)
-def test_weight_grad(gpu, shape):
-    """g.T @ x at the edges of a 64-row stage, a 256-column tile and a row split, against float64
+def test_linear_grads(gpu, shape):
+    """g.T @ x and the column sums of g at the edges of a 64-row stage, a 256-column tile and a row split, against float64
     (rounded once to bf16: 2^-9 of a value, 1.7e-3 of the norm; 3e-3 with the fp32 sums), from
     rows of wider tensors too, and bit for bit on a repeat."""
     M, N, K = shape
     g = torch.Generator().manual_seed(M + N + K)
     a, x = _bf((M, N + 8), g).to(gpu), _bf((M, K + 16), g).to(gpu)
     ref = a[:, :N].double().t() @ x[:, 16:].double()
-    got = ops.weight_grad(a[:, :N], x[:, 16:])
+    got, db = ops.linear_grads(a[:, :N], x[:, 16:], True)
     assert rel_l2(got.float().cpu(), ref.float().cpu()) <= 3e-3
-    assert torch.equal(got, ops.weight_grad(a[:, :N].contiguous(), x[:, 16:].contiguous()))
+    assert rel_l2(db.float().cpu(), a[:, :N].double().sum(0).float().cpu()) <= 3e-3
+    again, none = ops.linear_grads(a[:, :N].contiguous(), x[:, 16:].contiguous(), False)
+    assert torch.equal(got, again) and none.numel() == 0
+    assert torch.equal(db, ops.linear_grads(a[:, :N], x[:, 16:], True)[1])
 
 
-def test_weight_grad_second_derivative(gpu):
+def test_linear_grads_second_derivative(gpu):
     """create_graph through a Linear's weight gradient, against torch's own."""
     g = torch.Generator().manual_seed(5)
     x, w, v = _bf((40, 24), g), _bf((16, 24), g), _bf((16, 24), g)
