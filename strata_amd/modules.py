@@ -36,8 +36,8 @@ class GemmGeluMlp(nn.Module):
     screamcast/checkpoint_compat.py:243-249; GELU(tanh) per
     screamcast/strata_wrappers.py:76-100): fc1 + bias + GELU is one launch,
     fc2 + bias (+ the block's residual) another.  Under autograd (tanh GELU)
-    fc1's launch also writes gelu'(pre-activation),
-    which the backward multiplies by the upstream gradient.
+    fc1's launch also writes gelu'(pre-activation), which the backward multiplies
+    by the upstream gradient in the epilogue of its product with fc2's weight.
     """
 
     def __init__(self, in_features: int, hidden_features: int, out_features: Optional[int] = None,
@@ -64,6 +64,9 @@ class GemmGeluMlp(nn.Module):
     def forward(self, x: Tensor, residual: Optional[Tensor] = None) -> Tensor:
         fc1, act, fc2 = self.layers
         train = torch.is_grad_enabled() and (x.requires_grad or fc1.weight.requires_grad)
+        if train and act.approximate == "tanh" and not (fc1.in_features % 8 or fc1.out_features % 8
+                                                        or fc2.out_features % 8):
+            return ops.mlp_gelu_train(x, fc1.weight, fc1.bias, fc2.weight, fc2.bias, residual)[0]
         if train and act.approximate == "tanh":
             # fc1's launch also writes gelu'(pre-activation) for the backward (no recomputed GEMM)
             h, _ = ops.gemm_gelu_train(x, fc1.weight, fc1.bias)

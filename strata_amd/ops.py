@@ -29,6 +29,7 @@ __all__ = [
     "rope_qkv_pack",
     "gemm_bias_act",
     "gemm_gelu_train",
+    "mlp_gelu_train",
     "bias_grad",
     "linear_grads",
     "layer_norm",
@@ -336,10 +337,13 @@ def _na3d_lse_setup_context(ctx, inputs, output):
     out, lse = output
     ctx.kernel, ctx.dilation, ctx.scale = kernel, dilation, scale
     ctx.mark_non_differentiable(lse)
+    ctx.set_materialize_grads(False)  # no zero gradient of lse
     ctx.save_for_backward(q, k, v, out, lse)
 
 
 def _na3d_lse_backward(ctx, dout, dlse):
+    if dout is None:
+        return None, None, None, None, None, None
     q, k, v, out, lse = ctx.saved_tensors
     dq, dk, dv = na3d_bwd(q, k, v, out, dout.contiguous(), ctx.kernel, ctx.dilation, ctx.scale, lse)
     return dq, dk, dv, None, None, None
@@ -625,7 +629,7 @@ def _gemm_backward(ctx, dout):
     g2 = g.reshape(-1, g.shape[-1])
     x2 = x.reshape(-1, x.shape[-1])
     dx = (g2 @ w).reshape(x.shape) if ctx.needs_input_grad[0] else None
-    dw, db = _param_grads(ctx, g2, x2)
+    dw, db = _linear_param_grads(g2, x2, ctx.needs_input_grad[1], ctx.has_bias and ctx.needs_input_grad[2])
     if not gate:
         dres = dout if ctx.has_res and ctx.needs_input_grad[3] else None
     return dx, dw, db, dres, None, None
@@ -693,19 +697,86 @@ def _gelu_train_setup_context(ctx, inputs, output):
     _, dact = output
     ctx.has_bias = bias is not None
     ctx.mark_non_differentiable(dact)
+    ctx.set_materialize_grads(False)  # else a zero gradient of dact is filled and never read
     ctx.save_for_backward(x, w, dact)
 
 
 def _gelu_train_backward(ctx, dout, _ddact):
+    if dout is None:
+        return None, None, None
     x, w, dact = ctx.saved_tensors
     g2 = (dact * dout).reshape(-1, dact.shape[-1])  # the gradient at the pre-activation
     x2 = x.reshape(-1, x.shape[-1])
     dx = (g2 @ w).reshape(x.shape) if ctx.needs_input_grad[0] else None
-    dw, db = _param_grads(ctx, g2, x2)
+    dw, db = _linear_param_grads(g2, x2, ctx.needs_input_grad[1], ctx.has_bias and ctx.needs_input_grad[2])
     return dx, dw, db
 
 
 gemm_gelu_train.register_autograd(_gelu_train_backward, setup_context=_gelu_train_setup_context)
+
+
+@torch.library.custom_op("strata_hip::mlp_gelu_train", mutates_args=())
+def mlp_gelu_train(x: Tensor, w1: Tensor, b1: Optional[Tensor], w2: Tensor, b2: Optional[Tensor],
+                   residual: Optional[Tensor]) -> tuple[Tensor, Tensor, Tensor]:
+    """The MLP under autograd: ``out = gelu_tanh(x @ w1.T + b1) @ w2.T + b2 (+ residual)``, with
+    the hidden activations and the GELU's derivative at them (bf16) for the backward, whose
+    gradient at the hidden pre-activation is one launch (the product with w2 and, in its
+    epilogue, the derivative).  Every width a multiple of 8."""
+    name = "mlp_gelu_train"
+    _require_gpu(name, x, w1, b1, w2, b2, residual)
+    for t, nm in ((x, "x"), (w1, "w1"), (b1, "b1"), (w2, "w2"), (b2, "b2"), (residual, "residual")):
+        if t is not None and t.dtype != torch.bfloat16:
+            raise ValueError(f"{name}: {nm} must be bfloat16, got {t.dtype}")
+    K = x.shape[-1]
+    if w1.dim() != 2 or w2.dim() != 2 or w1.shape[1] != K or w2.shape[1] != w1.shape[0]:
+        raise ValueError(f"{name}: w1 must be [H, {K}] and w2 [N, H], got {tuple(w1.shape)}, {tuple(w2.shape)}")
+    H, N = w1.shape[0], w2.shape[0]
+    if K % 8 or H % 8 or N % 8:
+        raise ValueError(f"{name}: widths must be multiples of 8, got {K}, {H}, {N}")
+    for b, nm, n in ((b1, "b1", H), (b2, "b2", N)):
+        if b is not None and tuple(b.shape) != (n,):
+            raise ValueError(f"{name}: {nm} must be [{n}]")
+    if residual is not None and tuple(residual.shape) != (*x.shape[:-1], N):
+        raise ValueError(f"{name}: residual must have shape {(*x.shape[:-1], N)}, got {tuple(residual.shape)}")
+    h, dact = _gemm_gelu_train_launch(x, w1, b1)
+    return _gemm_launch(h, w2, b2, residual, _lib.ACT_NONE, _lib.RES_ADD), h, dact
+
+
+@mlp_gelu_train.register_fake
+def _(x, w1, b1, w2, b2, residual):
+    hidden = (*x.shape[:-1], w1.shape[0])
+    return x.new_empty((*x.shape[:-1], w2.shape[0])), x.new_empty(hidden), x.new_empty(hidden)
+
+
+def _mlp_train_setup_context(ctx, inputs, output):
+    x, w1, b1, w2, b2, residual = inputs
+    _, h, dact = output
+    ctx.has_b1, ctx.has_b2, ctx.has_res = b1 is not None, b2 is not None, residual is not None
+    ctx.mark_non_differentiable(h, dact)
+    ctx.set_materialize_grads(False)
+    ctx.save_for_backward(x, w1, w2, h, dact)
+
+
+def _mlp_train_backward(ctx, dout, _dh, _ddact):
+    if dout is None:
+        return None, None, None, None, None, None
+    x, w1, w2, h, dact = ctx.saved_tensors
+    need = ctx.needs_input_grad
+    g = dout.contiguous()
+    g2, h2, x2 = (t.reshape(-1, t.shape[-1]) for t in (g, h, x))
+    dw2, db2 = _linear_param_grads(g2, h2, need[3], ctx.has_b2 and need[4])
+    dx = dw1 = db1 = None
+    if need[0] or need[1] or (ctx.has_b1 and need[2]):
+        if torch.is_grad_enabled():  # create_graph: differentiable in dout
+            gz = dact.reshape(h2.shape) * (g2 @ w2)
+        else:
+            gz = _gemm_launch(g2, w2.t().contiguous(), None, dact.reshape(h2.shape), _lib.ACT_NONE, _lib.RES_MUL)
+        dw1, db1 = _linear_param_grads(gz, x2, need[1], ctx.has_b1 and need[2])
+        dx = (gz @ w1).reshape(x.shape) if need[0] else None
+    return dx, dw1, db1, dw2, db2, dout if ctx.has_res and need[5] else None
+
+
+mlp_gelu_train.register_autograd(_mlp_train_backward, setup_context=_mlp_train_setup_context)
 
 
 @torch.library.custom_op("strata_hip::bias_grad", mutates_args=())
@@ -791,10 +862,9 @@ def _linear_grads_backward(ctx, d, db):
 linear_grads.register_autograd(_linear_grads_backward, setup_context=_linear_grads_setup_context)
 
 
-def _param_grads(ctx, g2: Tensor, x2: Tensor) -> tuple[Optional[Tensor], Optional[Tensor]]:
-    """The weight's and the bias's gradients a GEMM op's backward owes (inputs 1 and 2), each
-    None where none is wanted; torch's products for widths the kernel does not take."""
-    want_w, want_b = ctx.needs_input_grad[1], ctx.has_bias and ctx.needs_input_grad[2]
+def _linear_param_grads(g2: Tensor, x2: Tensor, want_w: bool, want_b: bool) -> tuple[Optional[Tensor], Optional[Tensor]]:
+    """The weight's and the bias's gradients of a Linear, each None where none is wanted;
+    torch's products for widths the kernel does not take."""
     N, K = g2.shape[1], x2.shape[1]
     if want_w and N % 8 == 0 and K % 8 == 0:
         dw, db = linear_grads(g2, x2, want_b)

@@ -137,3 +137,28 @@ def test_linear_grads_second_derivative(gpu):
     got = second(lambda a, b: ops.gemm_bias_act(a, b, None, None, _lib.ACT_NONE), torch.bfloat16)
     ref = second(lambda a, b: F.linear(a, b), torch.float64)
     assert rel_l2(got.double().cpu(), ref.cpu()) <= 2e-2
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 8, 8), (300, 64, 256, 72), (4096, 256, 1024, 256)], ids=str)
+@pytest.mark.parametrize("frozen", [(), ("w2",), ("x", "w1", "b1")], ids=str)
+def test_mlp_train_autograd(gpu, shape, frozen):
+    """The MLP's one-op autograd against torch's in fp32 (1e-2, as the Mlp test above), with
+    every gradient, without fc2's weight's, and with fc2's and the residual's alone."""
+    M, K, H, N = shape
+    g = torch.Generator().manual_seed(M + H)
+    vals = dict(x=_bf((M, K), g), w1=_bf((H, K), g, K**-0.5), b1=_bf((H,), g), w2=_bf((N, H), g, H**-0.5),
+                b2=_bf((N,), g), r=_bf((M, N), g))
+    dout = _bf((M, N), g)
+    grads = []
+    for dt in (torch.bfloat16, torch.float32):
+        t = {k: v.to(gpu, dt).requires_grad_(k not in frozen) for k, v in vals.items()}
+        if dt == torch.bfloat16:
+            out = ops.mlp_gelu_train(*t.values())[0]
+        else:
+            out = F.linear(F.gelu(F.linear(t["x"], t["w1"], t["b1"]), approximate="tanh"), t["w2"], t["b2"]) + t["r"]
+        out.backward(dout.to(gpu, dt))
+        grads.append({k: v.grad for k, v in t.items()})
+    for k, a in grads[0].items():
+        assert (a is None) == (k in frozen)
+        if a is not None:
+            assert rel_l2(a.float().cpu(), grads[1][k].cpu()) <= 1e-2, k
