@@ -6,8 +6,9 @@ device.  There is no CPU or eager fallback: CPU tensors are rejected and a
 missing library raises.  Every op has a fake (meta) implementation so that
 ``torch.compile`` traces through it.  ``na3d_fwd`` (full-grid queries),
 ``gemm_bias_act`` (act none / GELU(tanh) with an added residual, and the
-sigmoid gate), ``layer_norm`` and ``rope_qkv_pack`` (with or without qk_norm)
-have backwards on HIP kernels; the other ops' autograd formulas raise.
+sigmoid gate), ``mlp_gelu_train``, ``layer_norm`` and ``rope_qkv_pack`` (with or
+without qk_norm) have backwards on HIP kernels (a Linear's plain input gradient is
+torch's product); the other ops' autograd formulas raise.
 """
 
 from __future__ import annotations
@@ -611,8 +612,8 @@ def _gemm_backward(ctx, dout):
     added (the MLP's fc1 -> GELU and fc2 + residual, attn.qkv and attn.proj + residual), and
     of the attention gate ``sigmoid(x @ w.T + bias) * residual``.
     The gradient at the pre-activation of a GELU layer, ``gelu'(x @ w.T + bias) * dout``,
-    recomputes the GEMM with that epilogue fused (hand-written kernel); the input and
-    weight gradients are plain GEMMs."""
+    recomputes the GEMM with that epilogue fused (hand-written kernel); the parameters'
+    gradients are ``linear_grads``, the input's a plain product."""
     gate = ctx.act == _lib.ACT_SIGMOID and ctx.has_res and ctx.res_op == _lib.RES_MUL
     if not gate and (ctx.act not in (_lib.ACT_NONE, _lib.ACT_GELU_TANH) or (ctx.has_res and ctx.res_op != _lib.RES_ADD)):
         raise RuntimeError("strata_hip::gemm_bias_act: backward covers act none / GELU(tanh) with an added "
