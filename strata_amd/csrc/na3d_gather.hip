@@ -32,7 +32,7 @@
 // head_dim 64 forward) times the union's share of useful pairs (49% at (3,7,7)).
 // Few tiles: SPLIT waves share one tile's rows and merge in LDS.  Measured, us,
 // a thread (backward: four lanes) per token -> here:
-//   fp32 forward  [1,4,16,16,4,32] (3,5,5)      135 -> 30 (a call; ~20 of it the host's)
+//   fp32 forward  [1,4,16,16,4,32] (3,5,5)      134 -> 8.9
 //   fp32 backward [1,16,64,64,8,64] (3,7,7)    7650 -> 1880 (forward 527, 37 TFLOP/s)
 //                 [1,8,64,64,8,128] (3,7,7)   12930 -> 1950
 //   bf16 backward [1,16,64,64,8,64] (3,7,7) dilation 2   2190 -> 893
