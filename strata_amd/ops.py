@@ -755,20 +755,22 @@ def _mlp_train_setup_context(ctx, inputs, output):
     ctx.has_b1, ctx.has_b2, ctx.has_res = b1 is not None, b2 is not None, residual is not None
     ctx.mark_non_differentiable(h, dact)
     ctx.set_materialize_grads(False)
-    ctx.save_for_backward(x, w1, w2, h, dact)
+    ctx.save_for_backward(x, w1, b1, w2, h, dact)
 
 
 def _mlp_train_backward(ctx, dout, _dh, _ddact):
     if dout is None:
         return None, None, None, None, None, None
-    x, w1, w2, h, dact = ctx.saved_tensors
+    x, w1, b1, w2, h, dact = ctx.saved_tensors
     need = ctx.needs_input_grad
+    if torch.is_grad_enabled():  # create_graph: the saved h carries no graph, so the hidden layer runs again
+        h, dact = gemm_gelu_train(x, w1, b1)
     g = dout.contiguous()
     g2, h2, x2 = (t.reshape(-1, t.shape[-1]) for t in (g, h, x))
     dw2, db2 = _linear_param_grads(g2, h2, need[3], ctx.has_b2 and need[4])
     dx = dw1 = db1 = None
     if need[0] or need[1] or (ctx.has_b1 and need[2]):
-        if torch.is_grad_enabled():  # create_graph: differentiable in dout
+        if torch.is_grad_enabled():  # products that autograd can go through
             gz = dact.reshape(h2.shape) * (g2 @ w2)
         else:
             gz = _gemm_launch(g2, w2.t().contiguous(), None, dact.reshape(h2.shape), _lib.ACT_NONE, _lib.RES_MUL)

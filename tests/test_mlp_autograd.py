@@ -1,0 +1,82 @@
+"""Autograd of the one-op MLP (``mlp_gelu_train``) without a GPU: its launches are replaced by
+torch products, so what is under test is the graph its backward builds."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from strata_amd import _lib, ops
+from strata_amd.modules import GemmGeluMlp
+
+from .conftest import rel_l2
+
+
+def _gelu_and_grad(z):
+    """gelu_tanh(z) and its derivative (an op's implementation runs below autograd: written out)."""
+    k = (2.0 / torch.pi) ** 0.5
+    t = torch.tanh(k * (z + 0.044715 * z**3))
+    return 0.5 * z * (1 + t), 0.5 * (1 + t) + 0.5 * z * (1 - t * t) * k * (1 + 3 * 0.044715 * z * z)
+
+
+@pytest.fixture
+def torch_launches(monkeypatch):
+    """The ops' launches on the CPU: fp32 products, each result rounded to bf16."""
+
+    def linear(x, w, b):
+        return F.linear(x.float(), w.float(), b.float() if b is not None else None)
+
+    def gemm(x, w, b, residual, act, res_op):
+        assert act == _lib.ACT_NONE
+        z = linear(x, w, b).bfloat16()
+        if residual is None:
+            return z
+        z = z.float() * residual.float() if res_op == _lib.RES_MUL else z.float() + residual.float()
+        return z.bfloat16()
+
+    def gelu_train(x, w, b):
+        h, d = _gelu_and_grad(linear(x, w, b))
+        return h.bfloat16(), d.bfloat16()
+
+    def linear_grads(g, x, bias):
+        return (g.float().t() @ x.float()).to(g.dtype), g.float().sum(0).to(g.dtype) if bias else g.new_empty(0)
+
+    monkeypatch.setattr(ops, "_require_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "_gemm_launch", gemm)
+    monkeypatch.setattr(ops, "_gemm_gelu_train_launch", gelu_train)
+    monkeypatch.setattr(ops, "linear_grads", linear_grads)
+
+
+def _second(m, x, residual, wrt, fixed_upstream):
+    """d |dW2|^2 / d(wrt): of loss = |out|^2, or with an upstream gradient that depends on nothing."""
+    out = m(x, residual)
+    up = None if not fixed_upstream else torch.ones_like(out)
+    loss = out if fixed_upstream else out.square().sum()
+    (dw2,) = torch.autograd.grad(loss, m.layers[2].weight, up, create_graph=True)
+    return torch.autograd.grad(dw2.square().sum(), wrt)
+
+
+class _Reference(torch.nn.Module):
+    def __init__(self, layers):
+        super().__init__()
+        self.layers = layers
+
+    def forward(self, x, residual):
+        return self.layers(x) + residual
+
+
+@pytest.mark.parametrize("fixed_upstream", [False, True])
+def test_second_derivative_reaches_the_hidden_layer(torch_launches, fixed_upstream):
+    """A penalty on fc2's weight gradient dY^T h reaches x, fc1's weight and bias through h, as in
+    float64 (bf16 roundings of out, h and each gradient in the chain: six of 2^-9, so 1.2e-2; a
+    path that is cut is off by a third or more)."""
+    torch.manual_seed(0)
+    m = GemmGeluMlp(24, 64, 16).bfloat16()
+    x, r = torch.randn(40, 24).bfloat16().requires_grad_(True), torch.randn(40, 16).bfloat16()
+    got = _second(m, x, r, [x, m.layers[0].weight, m.layers[0].bias], fixed_upstream)
+    ref = _Reference(torch.nn.Sequential(torch.nn.Linear(24, 64), torch.nn.GELU(approximate="tanh"),
+                                         torch.nn.Linear(64, 16))).double()
+    ref.load_state_dict({k: v.double() for k, v in m.state_dict().items()})
+    xd = x.detach().double().requires_grad_(True)
+    want = _second(ref, xd, r.double(), [xd, ref.layers[0].weight, ref.layers[0].bias], fixed_upstream)
+    for name, a, b in zip(("x", "w1", "b1"), got, want):
+        assert rel_l2(a, b) <= 1.2e-2, name

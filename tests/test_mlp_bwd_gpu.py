@@ -162,3 +162,22 @@ def test_mlp_train_autograd(gpu, shape, frozen):
         assert (a is None) == (k in frozen)
         if a is not None:
             assert rel_l2(a.float().cpu(), grads[1][k].cpu()) <= 1e-2, k
+
+
+def test_mlp_second_derivative(gpu):
+    """A penalty on the gradient of fc2's weight reaches x and fc1 through the hidden layer, on the
+    kernels (2e-2: the roundings of the chain, as for the Linear above)."""
+    g = torch.Generator().manual_seed(6)
+    vals = dict(x=_bf((40, 24), g), w1=_bf((64, 24), g, 24**-0.5), b1=_bf((64,), g), w2=_bf((16, 64), g, 64**-0.5),
+                b2=_bf((16,), g), r=_bf((40, 16), g))
+    grads = []
+    for dt in (torch.bfloat16, torch.float64):
+        t = {k: v.to(gpu, dt).requires_grad_(True) for k, v in vals.items()}
+        if dt == torch.bfloat16:
+            out = ops.mlp_gelu_train(*t.values())[0]
+        else:
+            out = F.linear(F.gelu(F.linear(t["x"], t["w1"], t["b1"]), approximate="tanh"), t["w2"], t["b2"]) + t["r"]
+        (dw2,) = torch.autograd.grad(out.square().sum(), t["w2"], create_graph=True)
+        grads.append(torch.autograd.grad(dw2.square().sum(), [t[k] for k in ("x", "w1", "b1")]))
+    for name, a, b in zip(("x", "w1", "b1"), *grads):
+        assert rel_l2(a.double().cpu(), b.cpu()) <= 2e-2, name
