@@ -773,7 +773,7 @@ def _mlp_train_backward(ctx, dout, _dh, _ddact):
         if torch.is_grad_enabled():  # products that autograd can go through
             gz = dact.reshape(h2.shape) * (g2 @ w2)
         else:
-            gz = _gemm_launch(g2, w2.t().contiguous(), None, dact.reshape(h2.shape), _lib.ACT_NONE, _lib.RES_MUL)
+            gz = gemm_bias_act(g2, w2.t().contiguous(), None, dact.reshape(h2.shape), _lib.ACT_NONE, _lib.RES_MUL)
         dw1, db1 = _linear_param_grads(gz, x2, need[1], ctx.has_b1 and need[2])
         dx = (gz @ w1).reshape(x.shape) if need[0] else None
     return dx, dw1, db1, dw2, db2, dout if ctx.has_res and need[5] else None

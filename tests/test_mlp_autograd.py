@@ -4,6 +4,7 @@ torch products, so what is under test is the graph its backward builds."""
 import pytest
 import torch
 import torch.nn.functional as F
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from strata_amd import _lib, ops
 from strata_amd.modules import GemmGeluMlp
@@ -80,3 +81,25 @@ def test_second_derivative_reaches_the_hidden_layer(torch_launches, fixed_upstre
     want = _second(ref, xd, r.double(), [xd, ref.layers[0].weight, ref.layers[0].bias], fixed_upstream)
     for name, a, b in zip(("x", "w1", "b1"), got, want):
         assert rel_l2(a, b) <= 1.2e-2, name
+
+
+@pytest.mark.parametrize("needs", [("x", "r", "layers.0.weight", "layers.0.bias", "layers.2.weight", "layers.2.bias"),
+                                   ("layers.0.weight", "layers.0.bias"), ("x",)], ids=["all", "fc1", "x"])
+def test_training_traces_without_data(needs):
+    """Forward and backward in one trace (what torch.compile of a training step does): every launch
+    in them is an op with a fake implementation, none asks a tensor without data for its pointer."""
+    m = GemmGeluMlp(24, 64, 16).bfloat16()
+    vals = dict(m.state_dict(), x=torch.randn(2, 20, 24).bfloat16(), r=torch.randn(2, 20, 16).bfloat16())
+
+    def step(vals):
+        vals = {k: t.detach().requires_grad_(k in needs) for k, t in vals.items()}
+        params = {k: t for k, t in vals.items() if "." in k}
+        out = torch.func.functional_call(m, params, (vals["x"], vals["r"]))
+        return torch.autograd.grad(out, [vals[k] for k in needs], torch.ones_like(out))
+
+    graph = make_fx(step, tracing_mode="fake")(vals)
+    names = [str(n.target) for n in graph.graph.nodes if "strata_hip" in str(n.target)]
+    assert "strata_hip.mlp_gelu_train.default" in names and "strata_hip.gemm_bias_act.default" in names
+    (outs,) = (n.args[0] for n in graph.graph.nodes if n.op == "output")
+    for k, n in zip(needs, outs):
+        assert n.meta["val"].shape == vals[k].shape and n.meta["val"].dtype == vals[k].dtype, k
