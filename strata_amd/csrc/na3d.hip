@@ -2331,7 +2331,7 @@ static int launch_f32(const Na3dParams& p, hipStream_t st) {
   g.scale = p.scale;
   g.lse = p.lse;
   g.lse_ext1 = p.lse_ext1;
-  return gather_fits(g, GATHER_FWD, 4) ? launch_gather(g, GATHER_FWD, false, st) : launch_scalar<float>(p, st);
+  return gather_plan(g, GATHER_FWD, 4) ? launch_gather(g, GATHER_FWD, false, st) : launch_scalar<float>(p, st);
 }
 
 // Query counts per axis of the box (largest over the dilation residue classes).

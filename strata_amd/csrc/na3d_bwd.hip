@@ -1649,8 +1649,8 @@ static int launch_bwd(const Na3dBwdParams& p, hipStream_t st) {
     hipLaunchKernelGGL((na3d_bwd_prep_kernel<T, D>), grid, block, 0, st, p);
   }
   if (!(sizeof(T) == 2 && D == 64 && mfma_ok(p)) && !std::getenv("STRATA_HIP_NA3D_BWD_VALU")) {
-    const GatherParams gq = bwd_gather(p, D, GATHER_DQ), gkv = bwd_gather(p, D, GATHER_DKV);
-    if (gather_fits(gq, GATHER_DQ, sizeof(T)) && gather_fits(gkv, GATHER_DKV, sizeof(T))) {
+    GatherParams gq = bwd_gather(p, D, GATHER_DQ), gkv = bwd_gather(p, D, GATHER_DKV);
+    if (gather_plan(gq, GATHER_DQ, sizeof(T)) && gather_plan(gkv, GATHER_DKV, sizeof(T))) {
       if (const int rc = launch_gather(gq, GATHER_DQ, sizeof(T) == 2, st)) return rc;
       return launch_gather(gkv, GATHER_DKV, sizeof(T) == 2, st);
     }

@@ -22,15 +22,16 @@ struct GatherParams {
   float* lse;         // forward: log2-sum-exp out or null; backward: the statistics read
   const float* dsum;  // backward: dO . O per query
   int lse_ext1;       // forward: y extent of the lse array
-  // set by the launch
+  // set by gather_plan
   int tl[3];    // log2 of the column tile's extent per axis, summing to 4
   int nt[3];    // tiles per axis (largest over the dilation residue classes)
   int nres, tiles;
 };
 
-// False: a shape or layout these kernels do not take (the caller keeps its general kernel).
-bool gather_fits(const GatherParams& p, int mode, int elem_bytes);
-// p as checked by gather_fits; bf16: T = bf16 (the backward), else float.
-int launch_gather(GatherParams p, int mode, bool is_bf16, hipStream_t st);
+// Sets the tile shape and counts.  False: a shape or layout these kernels do not take (the
+// caller keeps its general kernel).
+bool gather_plan(GatherParams& p, int mode, int elem_bytes);
+// p as gather_plan left it; bf16: T = bf16 (the backward), else float.
+int launch_gather(const GatherParams& p, int mode, bool is_bf16, hipStream_t st);
 
 }  // namespace strata

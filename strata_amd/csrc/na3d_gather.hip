@@ -38,6 +38,7 @@
 //   bf16 backward [1,16,64,64,8,64] (3,7,7) dilation 2   2190 -> 893
 //                 [1,8,40,52,8,32] (3,9,9)      877 -> 218
 //                 [1,16,64,64,8,64] (3,3,3) dilation 2    519 -> 436
+#include <cstdlib>
 #include <type_traits>
 
 #include "na3d_gather.h"
@@ -462,16 +463,21 @@ __global__ __launch_bounds__(256) void na3d_gather_kernel(GatherParams p) {
 #endif
 }
 
-// Most rows one column tile's union can hold along axis a.
-static int union_max(const GatherParams& p, int a, int t, int mode) {
-  const int sub = (p.L[a] + p.dil[a] - 1) / p.dil[a], k = p.ker[a];
-  // forward windows: k + t - 1; inverse windows reach at most 2 (k / 2) + 1 queries
-  // in the interior and k + k / 2 at a clamped edge
-  const int u = (mode == GATHER_DKV ? k + k / 2 : k) + t - 1;
-  return u < sub ? u : sub;
+// Most rows the union of a tile of t columns holds along axis a.  A window is k rows and
+// moves with its query: k + t - 1.  An inverse window is k rows in the interior and k / 2 more
+// where one end of the axis clamps; on an axis so short that one tile holds a key clamped at
+// the start (j < k) and one clamped at the end (j >= n - k), the union is the axis.
+static int64_t union_max(const GatherParams& p, int a, int t, int mode) {
+  const int64_t k = p.ker[a], d = p.dil[a];
+  auto rows = [&](int64_t n) -> int64_t {  // n: the length of a residue class
+    if (mode != GATHER_DKV) return n < k + t - 1 ? n : k + t - 1;
+    return n <= 2 * k + t - 2 ? n : k + k / 2 + t - 1;
+  };
+  const int64_t u0 = rows((p.L[a] + d - 1) / d), u1 = rows(p.L[a] / d);
+  return u0 > u1 ? u0 : u1;
 }
 
-bool gather_fits(const GatherParams& p, int mode, int elem_bytes) {
+bool gather_plan(GatherParams& p, int mode, int elem_bytes) {
   if (p.D != 32 && p.D != 64 && p.D != 128) return false;
   const int align = 16 / elem_bytes;  // every load and store of a token moves at most 16 bytes
   const void* ptrs[6] = {p.c0, p.c1 ? p.c1 : p.c0, p.s0, p.s1, p.o0, p.o1 ? p.o1 : p.o0};
@@ -481,19 +487,48 @@ bool gather_fits(const GatherParams& p, int mode, int elem_bytes) {
   for (const int64_t* s : strides)
     for (int i = 0; i < 5; ++i)
       if (s[i] % align) return false;
-  // table offsets are 32-bit, coordinates 10-bit
-  int64_t span0 = 0, span1 = 0;
-  int64_t tiles = (int64_t)p.B * p.H * p.dil[0] * p.dil[1] * p.dil[2];
+  int nq[3];
   for (int a = 0; a < 3; ++a) {
-    const int64_t u = union_max(p, a, 16, mode);
-    if (u > 1000) return false;
-    const int64_t d0 = p.ss0[1 + a] * p.dil[a], d1 = p.ss1[1 + a] * p.dil[a];
-    if (d0 > 0x3fffffff || d0 < -0x3fffffff || d1 > 0x3fffffff || d1 < -0x3fffffff) return false;
-    span0 += u * (d0 < 0 ? -d0 : d0);
-    span1 += u * (d1 < 0 ? -d1 : d1);
-    tiles *= p.ext[a];
+    nq[a] = 0;
+    for (int r = 0; r < p.dil[a]; ++r) {
+      const int c = sub_end(p.org[a], p.ext[a], r, p.dil[a]) - sub_first(p.org[a], r, p.dil[a]);
+      nq[a] = c > nq[a] ? c : nq[a];
+    }
   }
-  return span0 < 0x3fffffff && span1 < 0x3fffffff && tiles < 0x7fffffff;
+  p.nres = p.dil[0] * p.dil[1] * p.dil[2];
+  // The tile shape with the fewest row blocks over all tiles, of those whose union the row
+  // table describes: 10-bit coordinates, 32-bit element offsets.
+  int64_t best = INT64_MAX;
+  for (int lz = 0; lz <= 4; ++lz)
+    for (int ly = 0; ly + lz <= 4; ++ly) {
+      const int lg[3] = {lz, ly, 4 - lz - ly};
+      int64_t tiles = 1, rows = 1, span0 = p.D, span1 = p.D;
+      bool fits = true;
+      for (int a = 0; a < 3; ++a) {
+        const int64_t u = union_max(p, a, 1 << lg[a], mode);
+        const int64_t d0 = std::abs(p.ss0[1 + a] * p.dil[a]), d1 = std::abs(p.ss1[1 + a] * p.dil[a]);
+        tiles *= (nq[a] + (1 << lg[a]) - 1) >> lg[a];
+        rows *= u;
+        fits = u <= 1024 && d0 <= 0x7fffffff && d1 <= 0x7fffffff;
+        if (!fits) break;
+        span0 += (u - 1) * d0;
+        span1 += (u - 1) * d1;
+      }
+      if (!fits || span0 > 0x7fffffff || span1 > 0x7fffffff) continue;
+      const int64_t cost = tiles * ((rows + 15) / 16);
+      if (cost < best) {
+        best = cost;
+        for (int a = 0; a < 3; ++a) p.tl[a] = lg[a];
+      }
+    }
+  if (best == INT64_MAX) return false;
+  int64_t tiles = (int64_t)p.B * p.H * p.nres;
+  for (int a = 0; a < 3; ++a) {
+    p.nt[a] = (nq[a] + (1 << p.tl[a]) - 1) >> p.tl[a];
+    tiles *= p.nt[a];
+  }
+  p.tiles = (int)tiles;
+  return tiles <= 0x7ffffff0;
 }
 
 template <typename T, int D, int MODE>
@@ -518,34 +553,7 @@ static int launch_gather_d(const GatherParams& p, hipStream_t st) {
   }
 }
 
-int launch_gather(GatherParams p, int mode, bool is_bf16, hipStream_t st) {
-  int nq[3];
-  for (int a = 0; a < 3; ++a) {
-    nq[a] = 0;
-    for (int r = 0; r < p.dil[a]; ++r) {
-      const int c = sub_end(p.org[a], p.ext[a], r, p.dil[a]) - sub_first(p.org[a], r, p.dil[a]);
-      nq[a] = c > nq[a] ? c : nq[a];
-    }
-  }
-  p.nres = p.dil[0] * p.dil[1] * p.dil[2];
-  // the tile shape with the fewest row blocks over all tiles
-  int64_t best = INT64_MAX;
-  for (int lz = 0; lz <= 4; ++lz)
-    for (int ly = 0; ly + lz <= 4; ++ly) {
-      const int lg[3] = {lz, ly, 4 - lz - ly};
-      int64_t tiles = 1, rows = 1;
-      for (int a = 0; a < 3; ++a) {
-        tiles *= (nq[a] + (1 << lg[a]) - 1) >> lg[a];
-        rows *= union_max(p, a, 1 << lg[a], mode);
-      }
-      const int64_t cost = tiles * ((rows + 15) / 16);
-      if (cost < best) {
-        best = cost;
-        for (int a = 0; a < 3; ++a) p.tl[a] = lg[a];
-      }
-    }
-  for (int a = 0; a < 3; ++a) p.nt[a] = (nq[a] + (1 << p.tl[a]) - 1) >> p.tl[a];
-  p.tiles = p.B * p.H * p.nres * p.nt[0] * p.nt[1] * p.nt[2];
+int launch_gather(const GatherParams& p, int mode, bool is_bf16, hipStream_t st) {
   if (mode == GATHER_FWD) return launch_gather_d<float, GATHER_FWD>(p, st);
   if (mode == GATHER_DQ)
     return is_bf16 ? launch_gather_d<bf16, GATHER_DQ>(p, st) : launch_gather_d<float, GATHER_DQ>(p, st);

@@ -22,6 +22,7 @@ so those loops are evaluated at their first and last iteration.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass, field
 
@@ -425,6 +426,110 @@ def na3d_general_launch(B, L, H, ker, dil, qs, ks, vs, os_, org=(0, 0, 0), ext=N
                     inrec = (ten == tensor) & (voff + 16 <= col(nrec))
                     acc.add(name, col(base) + voff, 16, inrec)
     return acc
+
+
+class GatherParams(ctypes.Structure):
+    """na3d_gather.h GatherParams."""
+
+    _fields_ = [(n, ctypes.c_void_p) for n in ("c0", "c1", "s0", "s1", "o0", "o1")] + [
+        (n, ctypes.c_int) for n in "BHD"] + [(n, ctypes.c_int * 3) for n in ("L", "org", "ext", "ker", "dil")] + [
+        ("scale", ctypes.c_float)] + [(n, ctypes.c_int64 * 5) for n in ("cs", "ss0", "ss1", "os")] + [
+        ("lse", ctypes.c_void_p), ("dsum", ctypes.c_void_p), ("lse_ext1", ctypes.c_int), ("tl", ctypes.c_int * 3),
+        ("nt", ctypes.c_int * 3), ("nres", ctypes.c_int), ("tiles", ctypes.c_int)]
+
+
+GATHER_FWD, GATHER_DQ, GATHER_DKV = 0, 1, 2
+
+
+def gather_plan(lib, mode, B, L, H, D, ker, dil, strides, org=(0, 0, 0), ext=None, esize=4):
+    """The library's own choice of na3d_gather.hip's tiles (gather_plan): the planned
+    parameters, or None where it keeps the general kernel.  strides: of the columns, the
+    two row tensors and the output, elements (b, z, y, x, h)."""
+    p = GatherParams(B=B, H=H, D=D, L=tuple(L), org=tuple(org), ext=tuple(ext or L), ker=tuple(ker), dil=tuple(dil))
+    p.cs[:], p.ss0[:], p.ss1[:], p.os[:] = strides
+    plan = lib._ZN6strata11gather_planERNS_12GatherParamsEii
+    plan.argtypes, plan.restype = [ctypes.POINTER(GatherParams), ctypes.c_int, ctypes.c_int], ctypes.c_bool
+    return p if plan(p, mode, esize) else None
+
+
+def gather_launch(p: GatherParams, mode: int, esize: int = 4, pairs: bool = True):
+    """na3d_gather_kernel's index arithmetic at the planned parameters p: every global access of
+    one (b, h) = (0, 0) (the batch and head parts added at their extremes), and with pairs how
+    often each (column, row) pair of tokens is given weight, [columns, rows] over the grid."""
+    L, ker, dil, org, ext, tl, nt = (list(getattr(p, n)) for n in ("L", "ker", "dil", "org", "ext", "tl", "nt"))
+    acc = Access()
+    n_tok = L[0] * L[1] * L[2]
+    count = np.zeros((n_tok, n_tok), np.int32) if pairs else None
+    tok = lambda c: (c[0] * L[1] + c[1]) * L[2] + c[2]  # noqa: E731
+    bh = lambda s: np.array([0, (p.B - 1) * s[0] + (p.H - 1) * s[4]], np.int64) * esize  # noqa: E731
+
+    def window(j, n, k):  # first row and count of each column of the sub-grid
+        if mode != GATHER_DKV:
+            return _win_start(j, n, k), np.full_like(j, k)
+        r = k // 2
+        first = np.where(j - k + 1 <= 0, 0, j - k + 1 + r)
+        return first, np.where(j >= n - k, n - 1, j + r) - first + 1
+
+    for tile in range(p.nres * nt[0] * nt[1] * nt[2]):
+        w, tc, rg = tile, [0] * 3, [0] * 3
+        for a in (2, 1, 0):
+            tc[a], w = w % nt[a], w // nt[a]
+        res = w % p.nres
+        for a in (2, 1, 0):
+            rg[a], res = res % dil[a], res // dil[a]
+        li, lo, cnt, cc = np.arange(16), [0] * 3, [0] * 3, [0] * 3
+        u0, U, valid, live = [0] * 3, [0] * 3, np.ones(16, bool), True
+        for a in (2, 1, 0):
+            n = _sub_len(L[a], rg[a], dil[a])
+            q1 = _sub_end(org[a], ext[a], rg[a], dil[a])
+            q0 = _sub_first(org[a], rg[a], dil[a]) + (tc[a] << tl[a])
+            t, li = li & ((1 << tl[a]) - 1), li >> tl[a]
+            live &= q0 < q1
+            valid &= q0 + t < q1
+            f, _ = window(np.array([min(q0, max(q1 - 1, 0))]), n, ker[a])
+            u0[a] = int(f[0])
+            f, c = window(np.array([max(min(q0 + (1 << tl[a]) - 1, q1 - 1), 0)]), n, ker[a])
+            U[a] = int(f[0] + c[0]) - u0[a]
+            j = np.clip(q0 + t, 0, max(q1 - 1, 0))
+            f, cnt[a] = window(j, n, ker[a])
+            lo[a], cc[a] = f - u0[a], rg[a] + dil[a] * j
+        acc.add_sum("c", bh(p.cs), sum(cc[a] * p.cs[1 + a] for a in range(3)) * esize, p.D * esize)
+        if not live:
+            continue
+        f = np.arange(U[0] * U[1] * U[2])
+        xr, yr, zr = f % U[2], f // U[2] % U[1], f // U[2] // U[1]
+        for name, s in (("s0", p.ss0), ("s1", p.ss1)):
+            off = sum(c * dil[a] * s[1 + a] for a, c in enumerate((zr, yr, xr)))
+            acc.u32(f"{name} row offsets", off + p.D - 1, 1 << 31)
+            base = sum((rg[a] + dil[a] * u0[a]) * s[1 + a] for a in range(3))
+            acc.add_sum(name, bh(s), (base + off) * esize, p.D * esize)
+        packed = (zr | yr << 10 | xr << 20).astype(np.int64)
+        crd = [packed & 1023, packed >> 10 & 1023, packed >> 20]
+        oo = sum((cc[a] - org[a]) * p.os[1 + a] for a in range(3))
+        acc.add_sum("o", bh(p.os), oo[valid] * esize, p.D * esize)
+        if pairs:
+            rows = tok([rg[a] + dil[a] * (u0[a] + c) for a, c in enumerate((zr, yr, xr))])
+            held = np.ones((16, f.size), bool)
+            for a in range(3):
+                d = crd[a][None] - lo[a][:, None]
+                held &= (d >= 0) & (d < cnt[a][:, None])
+            cols = tok(cc)
+            for n in np.flatnonzero(valid):
+                np.add.at(count[cols[n]], rows[held[n]], 1)
+    return acc, count
+
+
+def window_pairs(L, ker, dil) -> np.ndarray:
+    """[queries, keys]: 1 where the query's clamped window holds the key (NATTEN's definition)."""
+    out = np.ones((1, 1), np.int32)
+    for n, k, d in zip(L, ker, dil):
+        m = np.zeros((n, n), np.int32)
+        for i in range(n):
+            g = i % d
+            start = int(_win_start(np.array(i // d), _sub_len(n, g, d), k))
+            m[i, g + d * np.arange(start, start + k)] = 1
+        out = np.kron(out, m)
+    return out
 
 
 def region_geom(KY: int) -> dict:

@@ -15,6 +15,8 @@ the scheme that breaks past 2^31 bytes) must be caught.
 import numpy as np
 import pytest
 
+from strata_amd import _lib
+
 from . import launch_model as LM
 
 
@@ -214,3 +216,57 @@ def test_upsample_dw_gelu_stays_inside_its_tensors(B, Z, Yc, Xc, C, f):
     assert lds == []
     assert acc.check({"cond": ncond, "out": nout, "weight": 2 * 9 * C}) == []
     assert acc.lo["out"] == 0 and acc.hi["out"] == nout
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _lib.load()
+
+
+# axis lengths around the places where inverse windows of a tile are clamped at both ends
+# (n = 2k + t - 2), dilated classes of unequal length, the column window, and a long window
+GATHER_GRIDS = [((1, 5, 1), (1, 3, 1), (1, 1, 1)), ((3, 9, 10), (3, 5, 5), (1, 1, 1)), ((1, 20, 21), (1, 9, 9), (1, 1, 1)),
+                ((1, 19, 33), (1, 3, 15), (1, 1, 1)), ((4, 11, 13), (3, 3, 3), (1, 2, 3)), ((6, 5, 7), (6, 1, 1), (1, 1, 1)),
+                ((2, 1, 90), (1, 1, 39), (1, 1, 1)), ((1, 1, 1300), (1, 1, 333), (1, 1, 1)),
+                ((1, 1022, 1), (1, 657, 1), (1, 1, 1)), ((1, 600, 2), (1, 401, 1), (1, 1, 1))]
+
+
+@pytest.mark.parametrize("mode", [LM.GATHER_FWD, LM.GATHER_DQ, LM.GATHER_DKV], ids=["fwd", "dq", "dkv"])
+@pytest.mark.parametrize("grid,ker,dil", GATHER_GRIDS, ids=str)
+def test_gather_kernel_pairs_and_bounds(lib, mode, grid, ker, dil):
+    """na3d_gather_kernel gives every (query, key) pair of a window its weight once and no other,
+    inside its tensors."""
+    st = LM.contiguous_strides([2, *grid, 3, 32])[:5]
+    p = LM.gather_plan(lib, mode, 2, grid, 3, 32, ker, dil, [st] * 4)
+    assert p is not None and sum(p.tl) == 4
+    acc, count = LM.gather_launch(p, mode)
+    size = 4 * 2 * int(np.prod(grid)) * 3 * 32
+    assert acc.check(dict.fromkeys(("c", "s0", "s1", "o"), size)) == []
+    assert acc.lo["o"] == 0 and acc.hi["o"] == size
+    want = LM.window_pairs(grid, ker, dil)
+    assert np.array_equal(count, want.T if mode == LM.GATHER_DKV else want)
+
+
+@pytest.mark.parametrize("n,k", [(1200, 657), (1025, 513), (1400, 1023)])
+def test_gather_kernel_refuses_unions_its_table_cannot_hold(lib, n, k):
+    """Inverse windows clamped at both ends of an axis reach all of it: past 1024 tokens the
+    coordinates of the row table would run into each other, so the general kernel stays."""
+    grid, ker = (1, n, 1), (1, k, 1)
+    st = LM.contiguous_strides([1, *grid, 1, 32])[:5]
+    assert LM.gather_plan(lib, LM.GATHER_DKV, 1, grid, 1, 32, ker, (1, 1, 1), [st] * 4) is None
+
+
+@pytest.mark.parametrize("fits,grid,ker,row", [
+    (True, (24, 144, 144), (3, 7, 7), 3 * 16 * 64),    # views of a packed qkv buffer
+    (True, (20, 256, 256), (3, 7, 7), 16 * 64),
+    (True, (24, 144, 144), (5, 7, 7), 16 * 1024),      # one z row apart fits, sixteen do not
+    (False, (24, 144, 144), (24, 7, 7), 16 * 1024),
+], ids=str)
+def test_gather_kernel_offsets_decide(lib, fits, grid, ker, row):
+    """The 32-bit row offsets of the tile that is launched decide, not those of the widest one."""
+    st = [grid[0] * grid[1] * grid[2] * row, grid[1] * grid[2] * row, grid[2] * row, row, 64]
+    p = LM.gather_plan(lib, LM.GATHER_FWD, 1, grid, 16, 64, ker, (1, 1, 1), [st, st, st, st])
+    assert (p is not None) == fits
+    if fits:
+        u = [min(n, k + (1 << t) - 1) for n, k, t in zip(grid, ker, p.tl)]
+        assert sum((a - 1) * s for a, s in zip(u, st[1:4])) + 64 <= 0x7FFFFFFF

@@ -221,6 +221,8 @@ def test_bwd_with_forward_lse_matches_recompute(gpu, case):
     ((6, 11, 17), 2, 64, (3, 3, 15), (1, 1, 1)),  # wider than the LDS kernels take
     ((4, 30, 33), 4, 128, (3, 7, 7), (1, 1, 1)),
     ((8, 18, 18), 1, 32, (7, 9, 9), (1, 1, 1)),   # more rows than one table holds
+    ((1, 1000, 1), 1, 32, (1, 555, 1), (1, 1, 1)),  # inverse windows of a whole long axis
+    ((1, 1200, 1), 1, 32, (1, 657, 1), (1, 1, 1)),  # one longer than the row table's coordinates
 ], ids=str)
 def test_bwd_gather_kernels(gpu, grid, H, D, kernel, dil, dtype, tol):
     """The fp32-arithmetic MFMA backward (fp32; bf16 with other head dims, dilation or wide

@@ -442,6 +442,21 @@ def test_fp32_gather_kernel(gpu, case, strided):
         assert (got_lse.cpu().double() - lse).abs().max().item() <= 1e-4
 
 
+def test_fp32_gather_kernel_row_offsets_past_two_to_the_30(gpu):
+    """A window whose rows lie more than 2^30 elements apart (z planes of 66 M elements, as a
+    packed qkv buffer of a large tile has them): the row table's offsets use all of 31 bits."""
+    L, H, D, kernel = (18, 6, 7), 2, 32, (17, 3, 5)
+    plane, row, tok = 66 << 20, 4096, 3 * H * D
+    buf = torch.empty(plane * L[0] + 8192, device=gpu)
+    strides = (plane * L[0], plane, row, tok, D, 1)
+    q, k, v = (buf.as_strided((1, *L, H, D), strides, i * H * D) for i in range(3))
+    ins = _rand((1, *L, H, D), 8, torch.float32, gpu)
+    for t, x in zip((q, k, v), ins):
+        t.copy_(x)
+    ref = O.na3d(*(t.cpu() for t in ins), kernel, compute_dtype=torch.float64)
+    assert (_run(q, k, v, kernel).cpu().double() - ref).abs().max().item() <= F32_TOL
+
+
 def test_fp32_gather_kernel_keeps_non_finite_values_inside_their_windows(gpu):
     """A NaN or infinite value token reaches exactly the queries whose windows hold it; a key of
     -inf scores carries no weight, and one of +inf or NaN scores makes its queries NaN."""
