@@ -331,7 +331,8 @@ int strata_hip_bias_grad(const strata_hip_bias_grad_args* args, void* stream);
  * the bias gradient bias_out[n] = sum over m of g[m, n].  n, k and the row strides
  * multiples of 8, 16-byte aligned pointers (bias_out: 2-byte).  workspace: fp32,
  * strata_hip_weight_grad_workspace(m, n, k, bias_out != NULL) elements (NULL when
- * that is 0).
+ * that is 0).  m at least 1; k == 0 with a bias_out is STRATA_HIP_EINVAL
+ * (strata_hip_bias_grad sums columns alone).
  * ------------------------------------------------------------------------- */
 typedef struct strata_hip_weight_grad_args {
   const void* g;

@@ -246,6 +246,8 @@ extern "C" int strata_hip_weight_grad(const strata_hip_weight_grad_args* a, void
   using namespace strata;
   if (!a) return fail(STRATA_HIP_EINVAL, "weight_grad: null args");
   if (a->m <= 0 || a->n < 0 || a->k < 0) return fail(STRATA_HIP_EINVAL, "weight_grad: bad m/n/k");
+  if (a->n > 0 && a->k == 0 && a->bias_out)
+    return fail(STRATA_HIP_EINVAL, "weight_grad: no columns of x (the column sums alone: strata_hip_bias_grad)");
   if (a->n == 0 || a->k == 0) return STRATA_HIP_OK;
   if (!a->g || !a->x || !a->out) return fail(STRATA_HIP_EINVAL, "weight_grad: null pointer");
   if (a->n % 8 || a->k % 8 || a->ldg % 8 || a->ldx % 8 || a->ldg < a->n || a->ldx < a->k)

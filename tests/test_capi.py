@@ -22,6 +22,7 @@ STRUCTS = {
     "strata_hip_rope_pack_args": _lib.RopePackArgs,
     "strata_hip_gemm_args": _lib.GemmArgs,
     "strata_hip_bias_grad_args": _lib.BiasGradArgs,
+    "strata_hip_weight_grad_args": _lib.WeightGradArgs,
     "strata_hip_layer_norm_args": _lib.LayerNormArgs,
     "strata_hip_cube_pad_args": _lib.CubePadArgs,
     "strata_hip_cube_crop_args": _lib.CubeCropArgs,
@@ -124,6 +125,29 @@ def test_bias_grad_validation_and_workspace(lib):
     assert "multiples of 8" in lib.strata_hip_last_error().decode()
     b.n, b.ldg, b.workspace = 16, 16, None
     assert lib.strata_hip_bias_grad(ctypes.byref(b), None) == _lib.EINVAL
+
+
+def test_weight_grad_validation_and_workspace(lib):
+    assert lib.strata_hip_weight_grad_workspace(64, 256, 256, 0) == 0  # one row range, straight to out
+    assert lib.strata_hip_weight_grad_workspace(65536, 768, 768, 0) == 28 * 768 * 768  # 9 tiles, 28 row ranges
+    assert lib.strata_hip_weight_grad_workspace(65536, 768, 768, 1) == 28 * 768 * 768 + 28 * 3 * 768
+    w = _lib.WeightGradArgs()
+    w.g = w.x = w.out = w.workspace = w.bias_out = 0x1000
+    w.m, w.n, w.k, w.ldg, w.ldx = 64, 16, 12, 16, 12
+    assert lib.strata_hip_weight_grad(ctypes.byref(w), None) == _lib.EINVAL
+    assert "multiples of 8" in lib.strata_hip_last_error().decode()
+    w.k = w.ldx = 16
+    w.workspace = None
+    assert lib.strata_hip_weight_grad(ctypes.byref(w), None) == _lib.EINVAL
+    assert "workspace" in lib.strata_hip_last_error().decode()
+    # no columns of x: nothing to write, unless column sums of g were asked for
+    w.k = w.ldx = 0
+    assert lib.strata_hip_weight_grad(ctypes.byref(w), None) == _lib.EINVAL
+    assert "bias_grad" in lib.strata_hip_last_error().decode()
+    w.bias_out = None
+    assert lib.strata_hip_weight_grad(ctypes.byref(w), None) == _lib.OK
+    w.n, w.k, w.bias_out = 0, 0, 0x1000
+    assert lib.strata_hip_weight_grad(ctypes.byref(w), None) == _lib.OK
 
 
 def test_gemm_and_layernorm_validation(lib):
