@@ -864,3 +864,290 @@ def cdiv(a, b):
 __all__ = ["Access", "OOB", "gemm_dma_launch", "gemm_sizes", "gemm_tile_origins", "layer_norm_launch",
            "rope_pack_half_launch", "na3d_general_launch", "na3d_column_launch", "production_block_launches", "span", "tensor_bytes",
            "contiguous_strides", "cdiv", "math"]
+
+
+# ---------------------------------------------------------------------------
+# GEMM, smaller tiles: gemm_tile_kernel<BM, BN, WGM, WGN, NST> (gemm.hip)
+# ---------------------------------------------------------------------------
+GEMM_TILES = {"128": (128, 128, 4, 2), "128 deep": (128, 128, 4, 2), "64": (64, 64, 2, 2)}
+
+
+def gemm_choose(M: int, N: int, K: int, cus: int = 256) -> str:
+    """gemm.hip gemm_choose: "256" or a key of GEMM_TILES."""
+    if N % 8:
+        return "256"
+    tiles = lambda b: cdiv(M, b) * cdiv(N, b)  # noqa: E731
+    r = tiles(256) / cus
+    whole, part = int(r), r - int(r)
+    cost = {"256": 3000.0 + whole * (26.0 * K + 5000.0) + ((16.5 + 9.5 * part) * K + 5000.0 if part > 0 else 0.0)}
+    r128, r64 = tiles(128) / (2.0 * cus), tiles(64) / (2.0 * cus)
+    cost["128"] = 3000.0 + r128 * (17.9 * K + 3700.0) if r128 > 1 else 4000.0 + (8.3 + 9.6 * r128) * K
+    if r128 <= 0.5:
+        cost["128 deep"] = 3000.0 + (7.0 + 5.2 * r128) * K
+    cost["64"] = 2000.0 + r64 * (7.05 * K + 1600.0) if r64 > 1 else 2000.0 + (5.0 + 2.0 * r64) * K
+    return min(cost, key=cost.get)
+
+
+def gemm_tile_launch(tile: str, M: int, N: int, K: int, ldx: int, ldw: int, ldo: int, ldr: int | None = None,
+                     bias: bool = False, save: bool = False) -> tuple[Access, np.ndarray]:
+    """Every global access of one gemm_tile_kernel launch (the copies' lane offsets voff and the
+    masked last stage, the bias quads, the epilogue's 16-byte rows), lane by lane, and how often
+    each 8-element run of the output is written [M, N / 8]."""
+    BM, BN, WGM, WGN = GEMM_TILES[tile]
+    NW, WTM, WTN = WGM * WGN, BM // WGM, BN // WGN
+    xch, lpw = BM * 128 // 1024, (BM + BN) * 128 // 1024 // NW
+    acc, mt, nt = Access(), cdiv(M, BM), cdiv(N, BN)
+    acc.u32("workgroups", [mt * nt], 1 << 31)
+    wg = _xcd_order(mt * nt, np.arange(mt * nt, dtype=np.int64))
+    gi, li = wg // (8 * nt), wg % (8 * nt)
+    gmn = np.minimum(8, mt - gi * 8)
+    m0, n0 = ((gi * 8 + li % gmn) * BM)[:, None, None], ((li // gmn) * BN)[:, None, None]
+    wave, lane = np.arange(NW)[None, :, None], np.arange(64)[None, None, :]
+    nk, ktail = cdiv(K, 64), K % 64
+    landed = np.zeros((BM + BN) * 128 // 16, np.int64)  # 16-byte pieces of a stage in LDS
+    for kt in sorted({0, nk - 1}):
+        for j in range(lpw):
+            isw = j * NW >= xch
+            row = 8 * (j * NW + wave - (xch if isw else 0)) + lane // 8
+            lc = _gswz8(lane % 8, row)
+            ok = ((n0 if isw else m0) + row < (N if isw else M)) & ~((kt == nk - 1) & (ktail > 0) & (lc * 8 >= ktail))
+            ld = ldw if isw else ldx
+            voff = np.where(ok, row * ld * 2 + lc * 16, OOB)
+            acc.lane_offsets("gemm tile", voff)
+            acc.add("w" if isw else "x", 2 * ((n0 if isw else m0) * ld + kt * 64) + voff, 16, ok)
+            if kt == 0:
+                np.add.at(landed, (wave * 64 + j * NW * 64 + lane).ravel(), 1)
+    assert (landed == 1).all()
+    wm, wn = wave // WGN, wave % WGN
+    gn0, gm0 = n0 + wn * WTN, m0 + wm * WTM
+    if bias:
+        for i in range(WTN // 32):
+            for q in range(4):
+                acc.add("bias", 2 * np.minimum(gn0 + 32 * i + 8 * q + 4 * (lane // 32), N - 4), 8)
+    cpr = WTN // 8
+    rpi = 64 // cpr
+    written = np.zeros((M, N // 8), np.int64)
+    outs = [("out", ldo)] + ([("res", ldr)] if ldr is not None else []) + ([("out2", ldo)] if save else [])
+    for it in range(WTM // rpi):
+        gm, gn = gm0 + rpi * it + lane // cpr, gn0 + 8 * (lane % cpr)
+        ok = (gn < N) & (gm < M)
+        for name, ld in outs:
+            acc.add(name, 2 * (gm * ld + gn), 16, ok)
+        gm, gn = np.broadcast_to(gm, ok.shape)[ok], np.broadcast_to(gn, ok.shape)[ok]
+        np.add.at(written, (gm, gn // 8), 1)
+    return acc, written
+
+
+# ---------------------------------------------------------------------------
+# Weight gradient (strata_amd/csrc/wgrad.hip)
+# ---------------------------------------------------------------------------
+def weight_grad_launch(M: int, N: int, K: int, ldg: int, ldx: int, bias: bool) -> tuple[Access, int, np.ndarray]:
+    """Both launches: weight_grad_kernel's copies, partials and column sums, and
+    weight_grad_finish_kernel's reads and stores.  Returns the accesses, the workspace's fp32
+    elements and how often each quad of each partial (or of the output) is written."""
+    acc, nt, kt = Access(), cdiv(N, 256), cdiv(K, 256)
+    tiles, stages = nt * kt, cdiv(M, 64)
+    want = min(max(256 // tiles, 1), max(stages // 4, 1))
+    per = cdiv(stages, want)
+    rows_per, splits = per * 64, cdiv(stages, per)
+    bfloats = cdiv(want * kt * N, 4) * 4 if bias else 0
+    ws = (want * N * K if want > 1 else 0) + bfloats
+    wave, lane = np.arange(8)[:, None], np.arange(64)[None, :]
+    written = np.zeros((splits if want > 1 else 1, N, K // 4), np.int64)
+    summed = np.zeros((nt, stages), np.int64)  # turns at the column sums, per stage of rows
+    bwritten = np.zeros((splits * kt, N), np.int64)
+    order = _xcd_order(tiles * splits, np.arange(tiles * splits))
+    assert sorted(order.tolist()) == list(range(tiles * splits))
+    for w in range(tiles * splits):
+        tk, r = w % kt, w // kt
+        tn, sp = r % nt, r // nt
+        k0, n0, m0 = tk * 256, tn * 256, sp * rows_per
+        rows = min(rows_per, M - m0)
+        assert rows > 0  # every range holds rows
+        nk = cdiv(rows, 64)
+        for st in sorted({0, nk - 1}):
+            left = rows - st * 64
+            for j in range(4):
+                row = 2 * (j * 8 + wave) + (lane >> 5)
+                c = (lane & 31) ^ ((row & 7) << 1)
+                for name, ld, o0, n in (("x", ldx, k0, K), ("g", ldg, n0, N)):
+                    ok = (o0 + 8 * c < n) & ~((left < 64) & (row >= left))
+                    voff = np.where(ok, row * ld * 2 + c * 16, OOB)
+                    acc.lane_offsets("weight_grad", voff)
+                    acc.add(name, 2 * ((m0 + st * 64) * ld + o0) + voff, 16, ok)
+        btick = tk
+        for st in range(nk):
+            if btick == 0:
+                summed[tn, m0 // 64 + st] += 1
+            btick = kt - 1 if btick == 0 else btick - 1
+        wk, wn, n16, g4 = wave >> 2, wave & 3, lane & 15, lane >> 4
+        for j in range(4):
+            n = n0 + 64 * wn + 16 * j + n16
+            if bias:
+                ok = (n < N) & (wk == 0) & (g4 == 0)
+                acc.add("ws", 4 * ((sp * kt + tk) * N + n), 4, ok)
+                np.add.at(bwritten, (sp * kt + tk, np.broadcast_to(n, ok.shape)[ok]), 1)
+            for i in range(8):
+                k = k0 + 128 * wk + 16 * i + 4 * g4
+                ok = (n < N) & (k < K)
+                if want > 1:
+                    acc.add("ws", 4 * (bfloats + (sp * N + n) * K + k), 16, ok)
+                else:
+                    acc.add("out", 2 * (n * K + k), 8, ok)
+                np.add.at(written, (sp if want > 1 else 0, np.broadcast_to(n, ok.shape)[ok],
+                                    np.broadcast_to(k, ok.shape)[ok] // 4), 1)
+    if bias:
+        assert (summed == 1).all() and (bwritten == 1).all()
+        acc.add("bias_out", np.array([0]), np.array([2 * N]))
+        acc.add("ws", np.array([0]), np.array([4 * splits * kt * N]))
+    if want > 1:  # the second launch: eight elements per thread of each partial
+        i = np.arange(0, N * K, 8)
+        acc.add("out", 2 * i, 16)
+        acc.add("ws", 4 * (bfloats + (splits - 1) * N * K + i), 32)
+    return acc, ws, written
+
+
+# ---------------------------------------------------------------------------
+# Rollout step I/O by quads (strata_amd/csrc/pipeline.hip)
+# ---------------------------------------------------------------------------
+def pipe_wide(C, grid, patch):
+    """pipe_wide's geometry: tokens per workgroup NX, LDS pitch KP, log2 of the lanes per run."""
+    pz, py, px = patch
+    Tx, K = grid[2] // px, C * pz * py * px
+    KP = (cdiv(K, 2) | 1) * 2
+    nx = 64 // px
+    while nx * px > 4 and nx * KP * 2 > 20480:
+        nx //= 2
+    assert px in (1, 2, 4) and grid[2] % 4 == 0 and nx * KP * 2 <= 64 * 1024
+    while nx * px > 4 and nx // 2 >= Tx:
+        nx //= 2
+    rql = 0
+    while 4 << rql < nx * px:
+        rql += 1
+    return nx, KP, rql
+
+
+def state_quads_launch(B, C, grid, patch, order=0) -> tuple[Access, dict]:
+    """state_patchify_wide_kernel and state_update_wide_kernel (order 0 or 1): the state quads
+    and the token pieces of each workgroup, the LDS elements used; how often each state quad
+    and each token element is moved."""
+    (Z, Y, X), (pz, py, px) = grid, patch
+    nx, KP, rql = pipe_wide(C, grid, patch)
+    Tz, Ty, Tx, K, rows = Z // pz, Y // py, X // px, C * pz * py * px, C * pz * py
+    magic = lambda d: cdiv(1 << 32, d) if d > 1 else 0  # noqa: E731
+    div = lambda n, d: (n * magic(d)) >> 32 if d > 1 else n  # noqa: E731
+    acc = Access()
+    quads = np.zeros((B, C, Z, Y, X // 4), np.int64)
+    lds = {}
+    tid = np.arange(256)
+    x, rr, step = 4 * (tid & ((1 << rql) - 1)), tid >> rql, 256 >> rql
+    r = rr[None, :] + step * np.arange(cdiv(rows, step))[:, None]  # every pass, as r0 + u * step
+    last = np.minimum(r, rows - 1)
+    c = div(last, pz * py)
+    q = last - c * pz * py
+    dz = div(q, py)
+    dy = q - dz * py
+    assert np.array_equal(c, last // (pz * py)) and np.array_equal(dz, q // py)
+    tokens = np.zeros((B, Tz, Ty, Tx), np.int64)
+    for b in range(B):
+        for tz in range(Tz):
+            for ty in range(Ty):
+                for xb in range(cdiv(Tx, nx)):
+                    tx0 = xb * nx
+                    nt = min(nx, Tx - tx0)
+                    on = np.broadcast_to(x < nt * px, r.shape)
+                    at = (((b * C + c) * Z + tz * pz + dz) * Y + ty * py + dy) * X + tx0 * px + x
+                    acc.add("state", 4 * at, 16, on)
+                    live = on & (r < rows)
+                    np.add.at(quads.ravel(), at[live] // 4, 1)
+                    for e in range(4):  # patchify's and update's LDS element of the quad's value e
+                        t, dx = (x + e) // px, (x + e) % px
+                        el = {"patchify": t * KP + last * px + dx,
+                              "update": t * KP + dx * (1 if order == 0 else C) +
+                              (last * px if order == 0 else (dz * py + dy) * px * C + c)}
+                        for name, v in el.items():
+                            assert ((v % KP < K) & (v // KP < nt))[on].all()
+                            key = (name, b, tz, ty, xb)
+                            lds.setdefault(key, []).append(v[live])
+                    tokens[b, tz, ty, tx0:tx0 + nt] += 1
+                    base = (((b * Tz + tz) * Ty + ty) * Tx + tx0) * K
+                    acc.add("tokens", np.array([2 * base]), 2 * nt * K)
+    for (name, *_), v in lds.items():  # each element of the tile once
+        v = np.concatenate(v)
+        assert len(np.unique(v)) == len(v), name
+    assert (quads == 1).all() and (tokens == 1).all()
+    return acc, {"state": 4 * B * C * Z * Y * X, "tokens": 2 * B * Z * Y * X * C}
+
+
+def dealias_patchify_launch(B, C, grid, patch, ny, nx_taps) -> tuple[Access, dict]:
+    """dealias_patchify_kernel: the state rows and columns each workgroup loads, the LDS floats
+    its two filters read (only ones that were loaded), the token elements it writes (each once)."""
+    (Z, Y, X), (pz, py, px) = grid, patch
+    Tz, Ty, Tx = Z // pz, Y // py, X // px
+    unit, nch = max(4, px), cdiv(X, 128)
+    runx = cdiv(cdiv(X, nch), unit) * unit
+    NX = runx // px
+    NTY, slices = min(4, Ty), C * pz
+    CB = 1
+    while CB * py * px < 64:
+        CB *= 2
+    rows = NTY * py
+    SR = rows + (ny - 1 if ny > 1 else 0)
+    XW = min(runx + (nx_taps - 1 if nx_taps > 1 else 0) + 6, X + 3) // 4 * 4
+
+    def size():
+        KP = (cdiv(CB * py * px, 2) | 1) * 2
+        return CB * (SR + rows) * XW * 4 + NTY * NX * KP * 2
+
+    while CB > 1 and (size() > 40 * 1024 or CB // 2 >= slices):
+        CB //= 2
+    assert size() <= 64 * 1024
+    acc, K = Access(), slices * py * px
+    written = np.zeros((B, Tz, Ty, Tx, K), np.int64)
+    loy, lox = (ny - 1) // 2, (nx_taps - 1) // 2
+    clamp = lambda v, hi: np.minimum(np.maximum(v, 0), hi)  # noqa: E731
+    for b in range(B):
+        for tz in range(Tz):
+            for ty0 in range(0, Ty, NTY):
+                nty = min(NTY, Ty - ty0)
+                r0 = ty0 * py if ny == 1 else int(clamp(py * ty0 - loy, Y - py))
+                r1 = (ty0 + nty) * py if ny == 1 else int(clamp(py * (ty0 + nty - 1) - loy + ny - 1, Y - py)) + py
+                assert r1 - r0 <= SR
+                for tx0 in range(0, Tx, NX):
+                    nt = min(NX, Tx - tx0)
+                    run, xo = nt * px, tx0 * px
+                    c0 = (xo if nx_taps == 1 else int(clamp(xo - lox, X - px))) & ~3
+                    c1 = xo + run if nx_taps == 1 else int(clamp(xo + run - px - lox + nx_taps - 1, X - px)) + px
+                    nq = cdiv(c1 - c0, 4)
+                    assert nq <= XW // 4 and run % 4 == 0
+                    for s0 in range(0, slices, CB):
+                        ns = min(CB, slices - s0)
+                        s = s0 + np.arange(ns)[:, None, None]
+                        row, col = np.arange(r0, r1)[None, :, None], c0 + 4 * np.arange(nq)[None, None, :]
+                        at = (((b * C + s // pz) * Z + tz * pz + s % pz) * Y + row) * X + col
+                        acc.add("state", 4 * at, 16)
+                        yo = np.arange(nty * py)
+                        j, u = ty0 + yo // py, yo % py
+                        for t in range(ny):  # the y filter's rows of A
+                            src = (clamp(py * j - loy + t, Y - py) + u if ny > 1 else ty0 * py + yo) - r0
+                            assert src.min() >= 0 and src.max() < r1 - r0
+                        for x in range(0, run, 4):  # the x filter's columns of G
+                            xa = xo + x
+                            ja, jb = xa & ~(px - 1), (xa + 3) & ~(px - 1)
+                            if nx_taps == 1:
+                                cols = xa + np.arange(4)
+                            elif ja - lox >= 0 and jb - lox + nx_taps - 1 <= X - px:
+                                cols = xa - lox + np.arange(nx_taps + 3)
+                                ref = [int(clamp((xa + e) // px * px - lox + t, X - px)) + (xa + e) % px
+                                       for t in range(nx_taps) for e in range(4)]
+                                assert ref == [int(cols[t + e]) for t in range(nx_taps) for e in range(4)]
+                            else:
+                                ia = xa + np.arange(4)[None, :]
+                                jx = ia & ~(px - 1)
+                                cols = clamp(jx - lox + np.arange(nx_taps)[:, None], X - px) + ia - jx
+                            assert cols.min() >= c0 and cols.max() < c0 + 4 * nq
+                        written[b, tz, ty0:ty0 + nty, tx0:tx0 + nt, s0 * py * px:(s0 + ns) * py * px] += 1
+                        base = (((b * Tz + tz) * Ty + ty0 + np.arange(nty)[:, None]) * Tx + tx0 + np.arange(nt)) * K
+                        acc.add("tokens", 2 * (base + s0 * py * px), 2 * ns * py * px)
+    assert (written == 1).all()
+    return acc, {"state": 4 * B * C * Z * Y * X, "tokens": 2 * B * Z * Y * X * C}
