@@ -829,6 +829,9 @@ extern "C" int strata_hip_dealias_patchify(const strata_hip_state_patchify_args*
     return fail(STRATA_HIP_EUNSUPPORTED,
                 "dealias_patchify: patch widths 1, 2 and 4, an x extent that is a multiple of 4 and a 16-byte aligned "
                 "state (else strata_hip_dealias_axis per axis and strata_hip_state_patchify)");
+  // No filter: the chain is the patchify alone, whose kernel has no LDS passes over the state
+  // and keeps what the normalisation overflows (the filters take it as 0).
+  if (ny == 1 && nx == 1) return strata_hip_state_patchify(a, stream);
   p.state = a->state;
   p.tokens = a->tokens;
   p.mean = a->mean;

@@ -249,3 +249,15 @@ def test_dealias_patchify_equals_the_chain(gpu, case, norm):
         if len(t) > 1:
             x, m, s = ops.dealias_axis(x, m, s, axis, patch[axis], t), None, None
     assert torch.equal(got, ops.state_patchify(x, m, s, patch))
+
+
+@pytest.mark.parametrize("patch", [(1, 1, 1), (2, 2, 2), (1, 3, 4)], ids=str)
+def test_dealias_patchify_without_filters_is_the_patchify(gpu, patch):
+    """One tap on both axes filters nothing: the plain patchify's tokens, a normalised value past
+    fp32's range (a vanishing std) kept as the patchify keeps it."""
+    _, xg = _state((2, 3, 4, 6, 24), 7, gpu)
+    m, s = torch.tensor([0.5, -1.0, 0.0], device=gpu), torch.tensor([0.7, 1e-38, 0.0], device=gpu)
+    got = ops.dealias_patchify(xg, m, s, patch, [1.0], [1.0])
+    ref = ops.state_patchify(xg, m, s, patch)
+    assert torch.isinf(ref).any()
+    assert torch.equal(got.nan_to_num(7.0, 8.0, 9.0), ref.nan_to_num(7.0, 8.0, 9.0))
