@@ -21,7 +21,10 @@
 // accumulator, so they run on the 16 x faster v_mfma_f32_16x16x32_bf16 (the scale
 // applied to the scores instead of the columns); the fp32 weights enter the second
 // product as two bf16 terms, w = hi + lo to 2^-17, two v_mfma_f32_16x16x16_bf16
-// in the place of four fp32 steps.
+// in the place of four fp32 steps.  The gradients' error against float64, over the
+// VALU kernels' with fp32 weights, at 24 drawn shapes (head_dim 32, 64, 128, dilation
+// 1, 2): 0.9998 .. 1.0003, mean 1.0000 (the bf16 outputs round 2^8 times coarser).
+// A weight that bf16 does not hold (infinite, NaN) takes the VALU branch in fp32.
 //
 // The union is a box per tile; its rows' offsets and coordinates go through a
 // table in LDS (512 rows at a time, built by the wave), which makes any window,
@@ -242,9 +245,11 @@ __global__ __launch_bounds__(256) void na3d_gather_kernel(GatherParams p) {
     // acc += rows^T x weights; in: bit r = row 4g + r lies in the column's window
     auto accumulate = [&](f32x4 (&o)[NB], const Quad (&r)[4][NJ], const float (&wt)[4], const T* s, const int* t,
                           int blk, int in) {
-      bool bad;  // some row value is not finite
+      bool bad;  // some row value is not finite, or (two terms of it: inf - inf) some bf16 weight
+      u32x2 hi = {0u, 0u};
       if constexpr (HALF) {
-        uint32_t x = 0;
+        hi = (u32x2){pack_bf16x2(wt[0], wt[1]), pack_bf16x2(wt[2], wt[3])};
+        uint32_t x = gather_max_exp(gather_max_exp(0, hi[0]), hi[1]);
 #pragma unroll
         for (int st = 0; st < 4; ++st)
 #pragma unroll
@@ -287,7 +292,6 @@ __global__ __launch_bounds__(256) void na3d_gather_kernel(GatherParams p) {
       }
       if constexpr (HALF) {
         typedef short s16x4 __attribute__((ext_vector_type(4)));
-        const u32x2 hi = {pack_bf16x2(wt[0], wt[1]), pack_bf16x2(wt[2], wt[3])};
         const u32x2 lw = {pack_bf16x2(wt[0] - bf16_lo(hi[0]), wt[1] - bf16_hi(hi[0])),
                           pack_bf16x2(wt[2] - bf16_lo(hi[1]), wt[3] - bf16_hi(hi[1]))};
 #pragma unroll

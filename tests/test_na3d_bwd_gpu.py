@@ -254,3 +254,46 @@ def test_bwd_gather_kernels_keep_non_finite_values_inside_their_windows(gpu):
     one = torch.zeros_like(held)
     one[at] = True
     assert torch.isnan(got[0][one]).all() and (got[0][~one] - clean[0][~one]).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "dout"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")], ids=str)
+@pytest.mark.parametrize("dtype,D,dil", [(torch.float32, 32, 1), (torch.float32, 64, 1), (torch.float32, 128, 2),
+                                         (torch.bfloat16, 32, 1), (torch.bfloat16, 64, 2), (torch.bfloat16, 128, 1)])
+def test_bwd_gather_kernels_non_finite_as_the_valu_kernels(gpu, monkeypatch, dtype, D, dil, bad, where):
+    """One value that is NaN or infinite in q, k, v or the output gradient: the matrix-core kernels
+    write NaN and each infinity exactly where the VALU kernels do (fp32 weights, window by window),
+    an infinite weight among them, and agree elsewhere."""
+    g = torch.Generator().manual_seed(11)
+    t = {n: torch.randn((1, 3, 12, 13, 2, D), generator=g).to(gpu, dtype) for n in ("q", "k", "v", "dout")}
+    t[where][0, 1, 5, 6, 1, 3] = bad
+    kernel, dils = [3, 5, 5], [1, dil, dil]
+    out, lse = ops.na3d_fwd_lse(t["q"], t["k"], t["v"], kernel, dils, None)
+    args = (t["q"], t["k"], t["v"], out, t["dout"], kernel, dils, None, lse)
+    got = ops.na3d_bwd(*args)
+    monkeypatch.setenv("STRATA_HIP_NA3D_BWD_VALU", "1")
+    for name, a, b in zip(("dq", "dk", "dv"), got, ops.na3d_bwd(*args)):
+        a, b = a.float(), b.float()
+        fin = torch.isfinite(b)
+        assert torch.equal(a[~fin].nan_to_num(7.0, 8.0, 9.0), b[~fin].nan_to_num(7.0, 8.0, 9.0)), name
+        assert torch.isfinite(a[fin]).all(), name
+        assert rel_l2(a[fin], b[fin]) <= (2e-6 if dtype == torch.float32 else 4e-3), name
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 1e-2)], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("grid,H,D,kernel,dil", [
+    ((4, 9, 10), 2, 128, (3, 5, 5), (1, 1, 1)),
+    ((5, 13, 15), 2, 32, (3, 5, 3), (1, 2, 3)),
+    ((6, 11, 17), 2, 64, (3, 3, 15), (1, 2, 1)),
+], ids=str)
+def test_bwd_valu_kernels(gpu, monkeypatch, grid, H, D, kernel, dil, dtype, tol):
+    """The kernels that take what the others refuse (here by the switch), against the float64
+    oracle, tolerances as the tests above."""
+    monkeypatch.setenv("STRATA_HIP_NA3D_BWD_VALU", "1")
+    g = torch.Generator().manual_seed(13)
+    q, k, v, do = (torch.randn((2, *grid, H, D), generator=g).to(dtype) for _ in range(4))
+    ref = O.na3d_backward(q, k, v, do, kernel, dil, compute_dtype=torch.float64)
+    out, lse = ops.na3d_fwd_lse(q.to(gpu), k.to(gpu), v.to(gpu), list(kernel), list(dil), None)
+    got = ops.na3d_bwd(q.to(gpu), k.to(gpu), v.to(gpu), out, do.to(gpu), list(kernel), list(dil), None, lse)
+    for name, a, b in zip(("dq", "dk", "dv"), got, ref):
+        assert rel_l2(a.float().cpu(), b) <= tol, name
