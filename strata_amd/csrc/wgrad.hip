@@ -221,7 +221,10 @@ __global__ __launch_bounds__(256) void weight_grad_finish_kernel(const float* __
 }
 
 // Splits of the rows: one workgroup per CU (the ring admits one), at least four
-// stages each.
+// stages each.  256, not the device's own count: the order of the sums is the
+// shape's alone.  From 129 tiles on one split leaves CUs idle (144 of 256 at
+// 6144 x 1536) and more take more rounds and 190 MB of partials; the caller keeps
+// such shapes on torch's product where that is faster (ops._weight_grad_pays).
 static int wgrad_splits(int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((n + 255) / 256) * ((k + 255) / 256), stages = (m + WG_BK - 1) / WG_BK;
   int64_t s = tiles >= 256 ? 1 : 256 / tiles;

@@ -865,11 +865,32 @@ def _linear_grads_backward(ctx, d, db):
 linear_grads.register_autograd(_linear_grads_backward, setup_context=_linear_grads_setup_context)
 
 
+def _weight_grad_pays(M: int, N: int, K: int, bias: bool) -> bool:
+    """Whether ``linear_grads`` is at least as fast as torch's product (with ``bias_grad``).
+    Its workgroups are the 256 x 256 tiles of [N, K] times a split of the rows over 256 CUs, and
+    a second launch adds the splits.  Measured, us, kernel / torch:
+
+    * 129 to 160 tiles leave 3 of 8 CUs idle: N x K = 6144 x 1536, 16384 rows 368 / 328, 65536
+      rows 1529 / 1252; 2816 x 3072, 4096 rows 104 / 96 (16384 rows 367 / 431, given up); from
+      161 on 0.96 to 1.06 of torch's with a bias, 0.93 to 1.0 without, from 196 on faster.
+    * without a bias the second launch counts where few rows are split: 4096 x 1024, 1000 rows
+      34 / 23, 4096 rows 50 / 46, 8192 rows 77 / 86; up to 448 rows there is no split (19 / 20),
+      few tiles pay from 4096 rows on (512 x 128: 23 / 33)."""
+    tiles = -(-N // 256) * -(-K // 256)
+    if bias:
+        return not (128 < tiles <= 160 and M >= 2048)
+    if M <= 448:
+        return True
+    if M < 8192:
+        return (tiles >= 196 and M >= 2048) or (tiles < 16 and M >= 4096)
+    return not 128 < tiles < 196
+
+
 def _linear_param_grads(g2: Tensor, x2: Tensor, want_w: bool, want_b: bool) -> tuple[Optional[Tensor], Optional[Tensor]]:
     """The weight's and the bias's gradients of a Linear, each None where none is wanted;
-    torch's products for widths the kernel does not take."""
-    N, K = g2.shape[1], x2.shape[1]
-    if want_w and N % 8 == 0 and K % 8 == 0:
+    torch's products for widths the kernel does not take and sizes at which it is slower."""
+    (M, N), K = g2.shape, x2.shape[1]
+    if want_w and N % 8 == 0 and K % 8 == 0 and _weight_grad_pays(M, N, K, want_b):
         dw, db = linear_grads(g2, x2, want_b)
         return dw, db if want_b else None
     dw = g2.t() @ x2 if want_w else None

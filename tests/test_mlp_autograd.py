@@ -103,3 +103,21 @@ def test_training_traces_without_data(needs):
     (outs,) = (n.args[0] for n in graph.graph.nodes if n.op == "output")
     for k, n in zip(needs, outs):
         assert n.meta["val"].shape == vals[k].shape and n.meta["val"].dtype == vals[k].dtype, k
+
+
+@pytest.mark.parametrize("M,N,K,bias,kernel", [
+    (65536, 6144, 1536, True, False), (2048, 1536, 6144, True, False), (1000, 6144, 1536, True, True),
+    (65536, 4608, 1536, True, True), (65536, 3584, 3584, True, True), (65536, 3072, 768, True, True),
+    (1000, 4096, 1024, False, False), (1000, 4096, 1024, True, True), (256, 4096, 1024, False, True),
+    (4096, 2048, 2048, False, False), (4096, 512, 128, False, True), (8192, 2048, 2048, False, True),
+    (65536, 6144, 1536, False, False), (1000, 12, 64, True, False)])
+def test_weight_gradient_route(monkeypatch, M, N, K, bias, kernel):
+    """The weight gradient's kernel runs where it is the faster one, torch's product elsewhere
+    (no data: the route alone)."""
+    calls = []
+    monkeypatch.setattr(ops, "linear_grads", lambda g, x, b: (calls.append("kernel"), (g.t() @ x, g.sum(0)))[1])
+    monkeypatch.setattr(ops, "bias_grad", lambda g: g.sum(0))
+    g, x = (torch.empty(s, device="meta", dtype=torch.bfloat16) for s in ((M, N), (M, K)))
+    dw, db = ops._linear_param_grads(g, x, True, bias)
+    assert bool(calls) == kernel
+    assert tuple(dw.shape) == (N, K) and (db is not None) == bias
