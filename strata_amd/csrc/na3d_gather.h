@@ -31,6 +31,7 @@ struct GatherParams {
 // Sets the tile shape and counts.  False: a shape or layout these kernels do not take (the
 // caller keeps its general kernel).
 bool gather_plan(GatherParams& p, int mode, int elem_bytes);
+int gather_split(const GatherParams& p);
 // p as gather_plan left it; bf16: T = bf16 (the backward), else float.
 int launch_gather(const GatherParams& p, int mode, bool is_bf16, hipStream_t st);
 

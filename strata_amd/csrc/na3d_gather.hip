@@ -535,12 +535,21 @@ bool gather_plan(GatherParams& p, int mode, int elem_bytes) {
   return tiles <= 0x7ffffff0;
 }
 
+// Waves that share one tile's rows.  8 waves per CU hide the loads (two per SIMD); a problem with
+// fewer tiles splits each over 2 or 4.  The parts' sums are merged, so the split shows in the last
+// bits: it goes by the tiles of one sample, and a sample's result does not depend on its batch.
+// That costs batches of small samples up to a fifth against the split for the whole call: us at
+// 1 / 4 / 16 samples of [4,16,16,4,32] (3,5,5), 256 tiles, fp32 backward 31 / 42 / 110 (whole
+// call 31 / 38 / 101); of [8,24,24,4,128] (3,5,5), 1152 tiles, forward 47 / 142 / 562 (47 / 129 / 482).
+int gather_split(const GatherParams& p) {
+  constexpr int WANT = 2048;
+  const int tiles = p.tiles / p.B;
+  return tiles >= WANT ? 1 : tiles >= WANT / 2 ? 2 : 4;
+}
+
 template <typename T, int D, int MODE>
 static int launch_gather_t(const GatherParams& p, hipStream_t st) {
-  // Waves wanted: 8 per CU hide the loads (two per SIMD); a problem with fewer
-  // tiles splits each tile's rows over 2 or 4 waves.
-  constexpr int WANT = 2048;
-  const int split = p.tiles >= WANT ? 1 : p.tiles >= WANT / 2 ? 2 : 4;
+  const int split = gather_split(p);
   const dim3 grid((unsigned)((p.tiles + 4 / split - 1) / (4 / split))), block(256);
   if (split == 1) hipLaunchKernelGGL((na3d_gather_kernel<T, D, MODE, 1>), grid, block, 0, st, p);
   else if (split == 2) hipLaunchKernelGGL((na3d_gather_kernel<T, D, MODE, 2>), grid, block, 0, st, p);

@@ -12,6 +12,8 @@ every output tile exactly once, so the model follows the kernels.  A planted
 the scheme that breaks past 2^31 bytes) must be caught.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -270,3 +272,15 @@ def test_gather_kernel_offsets_decide(lib, fits, grid, ker, row):
     if fits:
         u = [min(n, k + (1 << t) - 1) for n, k, t in zip(grid, ker, p.tl)]
         assert sum((a - 1) * s for a, s in zip(u, st[1:4])) + 64 <= 0x7FFFFFFF
+
+
+@pytest.mark.parametrize("mode", [LM.GATHER_FWD, LM.GATHER_DQ, LM.GATHER_DKV], ids=["fwd", "dq", "dkv"])
+@pytest.mark.parametrize("grid,ker", [((4, 16, 16), (3, 5, 5)), ((8, 40, 52), (3, 9, 9)), ((16, 64, 64), (3, 7, 7))])
+def test_gather_kernel_sums_do_not_depend_on_the_batch(lib, mode, grid, ker):
+    """The tile and the number of waves that share its rows fix the order of a token's sums: the
+    same for a sample alone and inside any batch."""
+    st = LM.contiguous_strides([1, *grid, 4, 32])[:5]
+    split = lib._ZN6strata12gather_splitERKNS_12GatherParamsE
+    split.argtypes, split.restype = [ctypes.POINTER(LM.GatherParams)], ctypes.c_int
+    plans = [LM.gather_plan(lib, mode, b, grid, 4, 32, ker, (1, 1, 1), [st] * 4) for b in (1, 2, 5, 8, 64)]
+    assert len({(tuple(p.tl), split(p)) for p in plans}) == 1

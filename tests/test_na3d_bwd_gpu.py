@@ -236,6 +236,23 @@ def test_bwd_gather_kernels(gpu, grid, H, D, kernel, dil, dtype, tol):
         assert rel_l2(a.float().cpu(), b) <= tol, name
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_gather_kernels_do_not_depend_on_the_batch(gpu, dtype):
+    """A sample's output, statistics and gradients bit for bit alone and in a batch of 8."""
+    g = torch.Generator().manual_seed(12)
+    q, k, v, do = (torch.randn((8, 4, 16, 16, 4, 32), generator=g).to(gpu, dtype) for _ in range(4))
+    kernel, dil = [3, 5, 5], [1, 1, 1]
+
+    def run(*t):
+        out, lse = ops.na3d_fwd_lse(*t[:3], kernel, dil, None)
+        return (out, lse, *ops.na3d_bwd(*t[:3], out, t[3], kernel, dil, None, lse))
+
+    whole = run(q, k, v, do)
+    for b in (0, 7):
+        for name, a, w in zip(("out", "lse", "dq", "dk", "dv"), run(*(t[b:b + 1] for t in (q, k, v, do))), whole):
+            assert torch.equal(a[0], w[b]), name
+
+
 def test_bwd_gather_kernels_keep_non_finite_values_inside_their_windows(gpu):
     """A NaN output gradient at one query reaches dk and dv of exactly its window's keys."""
     g = torch.Generator().manual_seed(10)
