@@ -8,6 +8,7 @@ from oracle import rope as R
 from strata_amd import _lib, ops  # noqa: F401
 from strata_amd import rope as P
 
+from . import launch_model
 from .conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -435,6 +436,32 @@ def test_gemm_smaller_tiles(gpu, shape, act, res_op):
         bb = torch.cat([on(b), torch.zeros(n - N, dtype=torch.bfloat16, device=gpu)])
         rb = F.pad(rb, (0, n - N)) if rb is not None else None
         assert torch.equal(ops.gemm_bias_act(xb, wb, bb, rb, act, res_op or 0)[:M, :N], got)
+
+
+ALL_ACTS = [_lib.ACT_NONE, _lib.ACT_GELU_TANH, _lib.ACT_GELU_ERF, _lib.ACT_SIGMOID, _lib.ACT_GELU_TANH_GRAD,
+            _lib.ACT_SIGMOID_GRAD]
+
+
+@pytest.mark.parametrize("shape", TILE_SHAPES, ids=str)
+def test_gemm_tile_never_shows_in_a_result(gpu, shape):
+    """Every activation and residual mode, and both outputs of the training fc1, on the tile that
+    the shape takes: bit for bit the same rows and columns inside a product on 256 x 256 tiles."""
+    M, N, K = shape
+    big, wide = 70000, -(-N // 1024) * 1024
+    assert launch_model.gemm_choose(big, wide, K) == "256" != launch_model.gemm_choose(M, N, K)
+    g = torch.Generator().manual_seed(M + N + K)
+    x, b, r = (torch.randn(s, generator=g).bfloat16().to(gpu) for s in ((M, K), (N,), (M, N)))
+    w = (torch.randn((N, K), generator=g) * K**-0.5).bfloat16().to(gpu)
+    xb, wb, bb, rb = F.pad(x, (0, 0, 0, big - M)), F.pad(w, (0, 0, 0, wide - N)), F.pad(b, (0, wide - N)), F.pad(
+        r, (0, wide - N, 0, big - M))
+    for act in ALL_ACTS:
+        for res_op in (None, _lib.RES_ADD, _lib.RES_MUL):
+            res = (None, None) if res_op is None else (r, rb)
+            got = ops.gemm_bias_act(x, w, b, res[0], act, res_op or 0)
+            ref = ops.gemm_bias_act(xb, wb, bb, res[1], act, res_op or 0)[:M, :N]
+            assert torch.equal(got, ref), (act, res_op)
+    for got, ref in zip(ops.gemm_gelu_train(x, w, b), ops.gemm_gelu_train(xb, wb, bb)):
+        assert torch.equal(got, ref[:M, :N])
 
 
 def _gelu_tanh_grad(t):
