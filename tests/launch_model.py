@@ -817,19 +817,27 @@ def contiguous_strides(shape):
     return list(reversed(st))
 
 
+def gemm_launch(M, N, K, ldx, ldw, ldo, ldr=None, bias=False, cus=256) -> Access:
+    """The GEMM on the tile its size takes."""
+    tile = gemm_choose(M, N, K, cus)
+    if tile == "256":
+        return gemm_dma_launch(M, N, K, ldx, ldw, ldo, ldr, bias, cus=cus)
+    return gemm_tile_launch(tile, M, N, K, ldx, ldw, ldo, ldr, bias)[0]
+
+
 def production_block_launches(B, Z, Y, X, C, H, kernel, mlp_ratio=4, gated=True, cus=256, depthwise=False):
     """(name, Access, sizes) of every hand-written launch of one StrataBlock forward
     at inference with qk-norm (strata_amd/modules.py StrataBlock.forward,
     FusedNA3DAttention.attention): LN, qkv GEMM, pack (q and k, v read from qkv),
     NA3D (the region or general kernel; with depthwise, the alternate block's
     column kernel over window (Z, 1, 1)), the gate GEMM, proj + residual, LN,
-    fc1 + GELU, fc2 + residual."""
+    fc1 + GELU, fc2 + residual; each GEMM on the tile its size takes."""
     D = C // H
     M = B * Z * Y * X
     F = int(C * mlp_ratio)
     out = []
     out.append(("layer_norm 1", layer_norm_launch(M, C, C, C), {"x": span(M, C, C), "out": span(M, C, C)}))
-    out.append(("qkv gemm", gemm_dma_launch(M, 3 * C, C, C, C, 3 * C, bias=True, cus=cus),
+    out.append(("qkv gemm", gemm_launch(M, 3 * C, C, C, C, 3 * C, bias=True, cus=cus),
                 gemm_sizes(M, 3 * C, C, C, C, 3 * C, bias=True)))
     out.append(("rope pack (q, k; qk-norm)", rope_pack_half_launch(B, Z, Y, X, H, D, 3 * C, 1),
                 {"qkv": span(M, 3 * C, 3 * C), "q": 2 * M * C, "k": 2 * M * C, "tables": 4 * B * Y * X * D // 2}))
@@ -845,14 +853,14 @@ def production_block_launches(B, Z, Y, X, C, H, kernel, mlp_ratio=4, gated=True,
     vsz = span(M, 3 * C, 3 * C) - 2 * 2 * C
     out.append((kname, acc, {"q": 2 * M * C, "k": 2 * M * C, "v": vsz, "out": 2 * M * C}))
     if gated:
-        out.append(("gate gemm (sigmoid, x residual)", gemm_dma_launch(M, C, C, C, C, C, C, bias=True, cus=cus),
+        out.append(("gate gemm (sigmoid, x residual)", gemm_launch(M, C, C, C, C, C, C, bias=True, cus=cus),
                     gemm_sizes(M, C, C, C, C, C, C, bias=True)))
-    out.append(("proj gemm + residual", gemm_dma_launch(M, C, C, C, C, C, C, bias=True, cus=cus),
+    out.append(("proj gemm + residual", gemm_launch(M, C, C, C, C, C, C, bias=True, cus=cus),
                 gemm_sizes(M, C, C, C, C, C, C, bias=True)))
     out.append(("layer_norm 2", layer_norm_launch(M, C, C, C), {"x": span(M, C, C), "out": span(M, C, C)}))
-    out.append(("fc1 gemm + gelu", gemm_dma_launch(M, F, C, C, C, F, bias=True, cus=cus),
+    out.append(("fc1 gemm + gelu", gemm_launch(M, F, C, C, C, F, bias=True, cus=cus),
                 gemm_sizes(M, F, C, C, C, F, bias=True)))
-    out.append(("fc2 gemm + residual", gemm_dma_launch(M, C, F, F, F, C, C, bias=True, cus=cus),
+    out.append(("fc2 gemm + residual", gemm_launch(M, C, F, F, F, C, C, bias=True, cus=cus),
                 gemm_sizes(M, C, F, F, F, C, C, bias=True)))
     return out
 
