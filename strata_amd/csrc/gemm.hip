@@ -737,7 +737,8 @@ __global__ __launch_bounds__(512, 1) void gemm_dma_kernel(GemmParams p) {
 // One BM x BN tile per workgroup of WGM x WGN waves; the stages of BK = 64
 // columns stream through an NST-slot LDS ring, NST - 1 stages ahead of the
 // MFMAs (a counted vmcnt wait leaves the younger stages' copies in flight).
-// Bound by the copies: a tile of half the edge moves twice the bytes per MFMA,
+// Bound by the copies: a tile of half the edge moves twice the bytes per MFMA (at
+// 10125 x 768 x 3072 waves wait 52% of the time, the matrix cores are busy 41%),
 // so these lose to the 256 x 256 kernel wherever that one fills the chip.
 // The MFMA, the K order and the bias as the first C operand are those of
 // gemm_dma_body, so the two agree bit for bit and the choice of a tile (which
@@ -1050,9 +1051,9 @@ static dim3 gemm_big(GemmParams& p) {
 //   64 x 64             2 per CU    5   .. 7        1.6
 // fitted on 40 shapes; the estimate picks the fastest of the four or one within
 // ~10% of it.  Measured, us, 256 x 256 only -> the choice: M x N x K =
-// 1024 x 256 x 1024 24.0 -> 7.6 (64 x 64), 2000 x 1024 x 4096 76 -> 28 (64 x 64),
-// 3040 x 888 x 3552 75 -> 34 (3 slots), 10125 x 768 x 3072 61 -> 52 (128 x 128),
-// 65536 x 128 x 128 15.9 -> 11.2 (128 x 128); at 49152 x 1024 x 4096 the 256 x 256
+// 1024 x 256 x 1024 24.0 -> 7.5 (64 x 64), 2000 x 1024 x 4096 76 -> 29 (64 x 64),
+// 3040 x 888 x 3552 75 -> 35 (3 slots), 10125 x 768 x 3072 61 -> 54 (128 x 128),
+// 65536 x 128 x 128 15.9 -> 11.5 (128 x 128); at 49152 x 1024 x 4096 the 256 x 256
 // kernel's 326 stand against 440 and 695.
 enum GemmTile { TILE_256, TILE_128, TILE_128_DEEP, TILE_64 };
 static GemmTile gemm_choose(const GemmParams& p) {

@@ -31,15 +31,17 @@
 // dilation and stride alike.  The tile's shape (16 = tz x ty x tx) is the one with
 // the fewest row blocks: 4 x 4 in y, x for square windows, 16 along z for (Z, 1, 1).
 //
-// Bound by the matrix cores' fp32 rate (1024 cycles per 16 x 16 block at
-// head_dim 64 forward) times the union's share of useful pairs (49% at (3,7,7)).
+// fp32 is bound by issue: at (3,7,7), head_dim 64 the matrix cores are busy for 46-50%
+// of the time (1024 cycles per 16 x 16 block forward, 49% of whose pairs are useful)
+// and the VALU for 28-52%, waves wait 13-17%.  bf16: VALU 56-58%, matrix cores 12-14%,
+// waves wait for the rows 32-42%.
 // Few tiles: SPLIT waves share one tile's rows and merge in LDS.  Measured, us,
 // a thread (backward: four lanes) per token -> here:
 //   fp32 forward  [1,4,16,16,4,32] (3,5,5)      134 -> 8.9
-//   fp32 backward [1,16,64,64,8,64] (3,7,7)    7650 -> 1880 (forward 527, 37 TFLOP/s)
-//                 [1,8,64,64,8,128] (3,7,7)   12930 -> 1950
-//   bf16 backward [1,16,64,64,8,64] (3,7,7) dilation 2   2190 -> 893
-//                 [1,8,40,52,8,32] (3,9,9)      877 -> 218
+//   fp32 backward [1,16,64,64,8,64] (3,7,7)    7650 -> 1850 (forward 525, 37 TFLOP/s)
+//                 [1,8,64,64,8,128] (3,7,7)   12930 -> 1950 .. 2140
+//   bf16 backward [1,16,64,64,8,64] (3,7,7) dilation 2   2190 -> 900
+//                 [1,8,40,52,8,32] (3,9,9)      877 -> 210
 //                 [1,16,64,64,8,64] (3,3,3) dilation 2    519 -> 436
 #include <cstdlib>
 #include <type_traits>

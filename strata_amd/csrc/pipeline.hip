@@ -406,12 +406,12 @@ static bool pipe_wide(PipeParams& p, const float* a, const float* b) {
 // reach are read once, normalised, into LDS; the y sums go to LDS; the x sums go
 // as bf16 into the token tile, which leaves like the patchify's.  The chain moved
 // the fp32 state five times; this reads it once (the taps' rows overlap in L2).
-// Bound by its instructions (the exact division of the normalisation, twice per
+// Bound by its instructions (VALU 88% busy: the exact division of the normalisation, twice per
 // element; the taps through LDS).  [6,80,16,64,64], patch 2 x 2, 5 taps: 367 us in
 // three launches -> 113.
 // ---------------------------------------------------------------------------
 // Per workgroup: four token rows, and channel slices for up to 64 elements of a
-// token in 40 KiB of LDS (three workgroups per CU).  Two or eight rows and 16 to
+// token in 40 KiB of LDS (four workgroups per CU or more).  Two or eight rows and 16 to
 // 128 elements measured 109-125 us at the shape above, patch 2 x 2 and 4 x 4.
 constexpr int DEALIAS_ROWS = 4, DEALIAS_KC = 64, DEALIAS_LDS = 40 * 1024;
 
