@@ -683,7 +683,11 @@ def _gemm_gelu_train_launch(x: Tensor, w: Tensor, bias: Optional[Tensor]) -> tup
     a.ldx, a.ldw = x2.stride(0) if M > 1 else K, w2.stride(0) if N > 1 else K
     a.ldr, a.ldo = 0, N
     a.act, a.res_op = _lib.ACT_GELU_TANH, _lib.RES_ADD
-    _launch("strata_hip_gemm_gelu_save", a, x, dact.data_ptr())
+    try:
+        _launch("strata_hip_gemm_gelu_save", a, x, dact.data_ptr())
+    except ValueError:  # every refusal of this call is the library's error, as a RuntimeError to recompute on
+        msg = _lib.load().strata_hip_last_error().decode(errors="replace")
+        raise _lib.StrataHipError("strata_hip_gemm_gelu_save", _lib.EINVAL, msg) from None
     return out, dact
 
 

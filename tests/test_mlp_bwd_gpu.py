@@ -181,3 +181,12 @@ def test_mlp_second_derivative(gpu):
         grads.append(torch.autograd.grad(dw2.square().sum(), [t[k] for k in ("x", "w1", "b1")]))
     for name, a, b in zip(("x", "w1", "b1"), *grads):
         assert rel_l2(a.double().cpu(), b.cpu()) <= 2e-2, name
+
+
+def test_gelu_train_refusals_are_the_librarys_error(gpu):
+    """K that is no multiple of 8: StrataHipError (a RuntimeError), from the op and the module."""
+    x, w = torch.zeros(4, 12, dtype=torch.bfloat16, device=gpu), torch.zeros(16, 12, dtype=torch.bfloat16, device=gpu)
+    with pytest.raises(_lib.StrataHipError, match="multiple of 8"):
+        ops.gemm_gelu_train(x, w, None)
+    with pytest.raises(_lib.StrataHipError, match="multiple of 8"):
+        GemmGeluMlp(12, 16, 8).to(gpu).bfloat16()(x.requires_grad_(True))
